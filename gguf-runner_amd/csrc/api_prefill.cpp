@@ -97,10 +97,15 @@ size_t prefill_f16_copy_bytes(const gr_prefill_args* a) {
     return align_up((size_t)rows * a->n_kv_heads * a->head_dim * 2, 256);
 }
 
-// [staging][K copy][V copy][flag, 256 B] for bf16, [staging] for f16.
+// [partials of a key-split launch][staging][K copy][V copy][flag, 256 B] for bf16,
+// [partials][staging] for f16.  The partials take the same room in every call, split
+// or not: a workspace sized for the longest chunk then also holds the shorter
+// chunks, which are the ones that split.
+size_t prefill_part_bytes(const gr_prefill_args* a) { return align_up(prefill_split_ws_bytes(a->head_dim), 256); }
 size_t prefill_ws_total(const gr_prefill_args* a) {
-    if (a->dtype != GR_DTYPE_BF16) return prefill_stage_bytes(a);
-    return prefill_stage_bytes(a) + 2 * prefill_f16_copy_bytes(a) + 256;
+    const size_t n = prefill_part_bytes(a) + prefill_stage_bytes(a);
+    if (a->dtype != GR_DTYPE_BF16) return n;
+    return n + 2 * prefill_f16_copy_bytes(a) + 256;
 }
 
 // Per-launch tag of the bf16 range flag: a launch reads "out of f16 range" only
@@ -149,11 +154,16 @@ int prefill_enqueue_ex(const gr_prefill_args* a, int in_dtype, hipStream_t st) {
     pp.v = a->v;
     pp.q_row_stride = (int64_t)a->n_heads * a->head_dim;
     pp.kv_row_stride = (int64_t)a->n_kv_heads * a->head_dim;
-    const bool fused = prefill_fused_q(a);
+    PrefillSplit split = prefill_split_plan(a->n_tokens, a->n_heads, a->n_kv_heads, a->head_dim, a->base_pos, a->window,
+                                            a->bidirectional ? 1 : 0);
+    pf_split_carve(split, a->n_kv_heads, a->workspace);
+    char* const stage = (char*)a->workspace + prefill_part_bytes(a);
+    // a split launch's workgroups each read their rows' Q: prepared once, by the prep pass
+    const bool fused = split.n_splits == 0 && prefill_fused_q(a);
     const bool bf16 = a->dtype == GR_DTYPE_BF16;
-    pp.q_out = fused ? nullptr : a->workspace;
+    pp.q_out = fused ? nullptr : stage;
     pp.q_out_lo = nullptr;
-    pp.rope_cs_out = fused && a->rope_mode != GR_ROPE_NONE ? (float*)a->workspace : nullptr;
+    pp.rope_cs_out = fused && a->rope_mode != GR_ROPE_NONE ? (float*)stage : nullptr;
     pp.q_out_dtype = GR_DTYPE_F16;  // bf16 caches too: the f16 path's operand (split exactly on the bf16 path)
     pp.q_out_scale = score_scale * 1.4426950408889634f;
     pp.k_cache = a->k_cache;
@@ -171,7 +181,7 @@ int prefill_enqueue_ex(const gr_prefill_args* a, int in_dtype, hipStream_t st) {
     uint32_t epoch = 0;
     hipError_t e = hipSuccess;
     if (bf16) {
-        char* w = (char*)a->workspace + prefill_stage_bytes(a);
+        char* w = stage + prefill_stage_bytes(a);
         k_f16 = (uint16_t*)w;
         v_f16 = (uint16_t*)(w + prefill_f16_copy_bytes(a));
         flag = (uint32_t*)(w + 2 * prefill_f16_copy_bytes(a));
@@ -239,6 +249,7 @@ int prefill_enqueue_ex(const gr_prefill_args* a, int in_dtype, hipStream_t st) {
         pf.f16_flag = flag;
         pf.f16_epoch = epoch;
     }
+    pf.split = split;
     e = launch_prefill(pf, st);
     if (e != hipSuccess) return hip_fail(e, "gr_prefill_attention launch");
     return GR_OK;

@@ -833,6 +833,9 @@ static int prefill_rows(gr_run_state* s, int32_t seq, int32_t layer, int64_t bas
         a.rope_dim = s->rope_dim;
         return a;
     };
+    auto q8_split = [&](int n, int64_t pos0) {
+        return prefill_q8_split_plan(n, s->cfg.n_heads, s->cfg.n_kv_heads, s->d, (int)pos0, (int)w, block ? 1 : 0);
+    };
     // Per piece: its rows' key ranges, the decode path's range arrays (uploaded
     // with the piece's rows) and the scratch its kernels carve; the pieces run in
     // stream order, so they share one scratch region.
@@ -849,7 +852,10 @@ static int prefill_rows(gr_run_state* s, int32_t seq, int32_t layer, int64_t bas
         pst[pc].assign(starts.begin() + r0, starts.begin() + r0 + n);
         pen[pc].assign(ends.begin() + r0, ends.begin() + r0 + n);
         size_t need = 4 * (size_t)n * s->q_dim + q8_stage_bytes(s, n) + 4 * 256;
-        if (!is_q8(s)) {
+        if (is_q8(s)) {
+            const PrefillSplit sp = q8_split(n, base_pos + r0);
+            need += pf_split_part_bytes(sp, s->cfg.n_kv_heads, s->d) + 256;
+        } else {
             gr_decode_args probe{};
             probe.n_seq = n;
             probe.n_heads = s->cfg.n_heads;
@@ -970,6 +976,8 @@ static int prefill_rows(gr_run_state* s, int32_t seq, int32_t layer, int64_t bas
             pq.v_scale = s->v_scale + so;
             pq.scale_row_stride = (int64_t)s->sc_per_row;
             pq.out = xi;
+            pq.split = q8_split(n, pos0);
+            pf_split_carve(pq.split, s->cfg.n_kv_heads, cw.take<char>(pf_split_part_bytes(pq.split, s->cfg.n_kv_heads, s->d)));
             const hipError_t e = launch_prefill_q8(pq, s->stream);
             return e == hipSuccess ? GR_OK : hip_fail(e, "q8 prefill launch");
         }

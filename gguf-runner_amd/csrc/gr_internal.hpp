@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "prefill_split.hpp"
+
 namespace gr {
 
 // Split-K decode.  Partials: ws_o [n_seq][n_heads][n_splits][head_dim],
@@ -302,7 +304,26 @@ struct PrefillLaunch {
     int64_t f16_row0, f16_row_stride;
     const uint32_t* f16_flag;
     uint32_t f16_epoch;
+    // n_splits > 0: key-split launch and combine (prefill_split.hpp); q prepared
+    // (q_raw null) at every head_dim
+    PrefillSplit split;
 };
+
+// The plan of a 16-bit prefill launch (n_splits 0: not split; partials unset),
+// and the bytes of partials that any plan of this head_dim needs at most.
+PrefillSplit prefill_split_plan(int n_tokens, int n_heads, int n_kv_heads, int head_dim, int base_pos, int window,
+                                int bidirectional);
+size_t prefill_split_ws_bytes(int head_dim);
+
+struct PrefillCombineLaunch {
+    int n_tokens, n_heads, n_kv_heads, head_dim;
+    int base_pos, window, bidirectional;
+    PrefillSplit split;
+    float* out;
+    OutGate gate;
+};
+
+hipError_t launch_prefill_combine(const PrefillCombineLaunch& p, hipStream_t st);
 
 hipError_t launch_prefill(const PrefillLaunch& p, hipStream_t st);
 
@@ -326,7 +347,12 @@ struct PrefillQ8Launch {
     int64_t scale_row_stride;
     float* out;
     OutGate gate;
+    PrefillSplit split;  // n_splits > 0: key-split launch and combine
 };
+
+// As prefill_split_plan; the partials take pf_split_part_bytes(plan, head_dim).
+PrefillSplit prefill_q8_split_plan(int n_tokens, int n_heads, int n_kv_heads, int head_dim, int base_pos, int window,
+                                   int bidirectional);
 
 hipError_t launch_prefill_q8(const PrefillQ8Launch& p, hipStream_t st);
 

@@ -18,7 +18,10 @@
 //                     B = P straight from the S^T accumulators)
 // so both accumulators hold one query per lane column and the online-softmax
 // statistics of a row live in the two lanes (l, l^32) that own it.
-// For head_dim 128 the kernel prepares Q itself from the raw rows (QK RMSNorm,
+// Launches whose workgroups would leave most CUs idle (short chunks over long
+// caches) are bound by one workgroup's chain of tiles; they are cut along the keys
+// (SPLIT, prefill_split.hpp) and finished by prefill_combine_kernel.
+// For head_dim 128 the unsplit kernel prepares Q itself from the raw rows (QK RMSNorm,
 // RoPE from a per-token (cos, sin) table, softmax_scale*log2(e)); otherwise Q
 // arrives prepared that way by the prep pass.
 #include <type_traits>
@@ -261,7 +264,9 @@ __device__ __forceinline__ void pf_prepare_q(const PrefillLaunch& p, int row, in
 // double-buffered tiles (BN * D each) and Qlo the bf16 d256 Q residuals, all in
 // LDS and declared by the kernel (distinct arrays, so the compiler sees that the
 // DMA into one buffer never aliases the reads of another).
-template <typename DT, int D, int NW, int KH = 1>
+// SPLIT: one piece of the keys of a block of packed rows (prefill_split.hpp), Q
+// prepared by the prep pass.
+template <typename DT, int D, int NW, int KH = 1, bool SPLIT = false>
 __device__ __forceinline__ void prefill_body(const PrefillLaunch& p, const void* k_cache, const void* v_cache,
                                              const int64_t rs, const int64_t row0, uint16_t* Ks0, uint16_t* Ks1,
                                              uint16_t* Vs0, uint16_t* Vs1, uint4* Qlo) {
@@ -292,20 +297,31 @@ __device__ __forceinline__ void prefill_body(const PrefillLaunch& p, const void*
     const int m = p.n_tokens;
     const int P0 = (int)p.base_pos;
     const int W = p.window;
-    const int n_qb = (m + BM - 1) / BM;
+    const int kv_mul = p.n_heads / p.n_kv_heads;
+    const int n_rows = SPLIT ? m * kv_mul : m;
+    const int n_qb = (n_rows + BM - 1) / BM;
     const int n_pairs = (n_qb + 1) / 2;
+    // token of a row (rows are packed (token, query head of the group) when SPLIT)
+    auto tok_of = [&](int r) { return SPLIT ? r / kv_mul : r; };
 
     // Work item = (query head, pair of query blocks), head-major.  Workgroup b
     // runs on XCD b % 8; giving each XCD a contiguous run of items keeps the
     // query heads of one GQA group (same K/V) in one XCD's L2.
+    // SPLIT: pf_split_item.
     const int n_items = p.n_heads * n_pairs;
     const int per_xcd = (n_items + 7) / 8;
     const int item = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-    if (item >= n_items) return;
-    const int h = item / n_pairs;
-    const int j = item - h * n_pairs;
-    const int kv_mul = p.n_heads / p.n_kv_heads;
-    const int g = h / kv_mul;
+    PfSplitItem si{0, 0, 0};
+    if constexpr (SPLIT) {
+        si = pf_split_item((int)blockIdx.x, p.n_kv_heads, p.split.n_qb, p.split.n_splits);
+        if (si.qb >= n_qb) return;
+    } else {
+        if (item >= n_items) return;
+    }
+    const int h = SPLIT ? 0 : item / n_pairs;
+    const int j = SPLIT ? si.qb : item - h * n_pairs;
+    const int piece = si.piece;
+    const int g = SPLIT ? si.g : h / kv_mul;
     const uint16_t* kc = (const uint16_t*)k_cache + (size_t)g * D;
     const uint16_t* vc = (const uint16_t*)v_cache + (size_t)g * D;
     const int rsb = (int)rs * 2;
@@ -339,19 +355,21 @@ __device__ __forceinline__ void prefill_body(const PrefillLaunch& p, const void*
         v_swz[b] = pf_swz<D>(r & 15);
     }
 
-    for (int pass = 0; pass < 2; pass++) {
-        const int qblk = pass == 0 ? n_qb - 1 - j : j;
+    for (int pass = 0; pass < (SPLIT ? 1 : 2); pass++) {
+        const int qblk = SPLIT ? j : pass == 0 ? n_qb - 1 - j : j;
         if (pass == 1 && qblk >= n_qb - 1 - j) break;
 
         const int q0 = qblk * BM;
         const int wr0 = q0 + rw * 32;
         const int my_row = wr0 + ln;
-        const bool row_ok = my_row < m;
-        const int my_row_c = row_ok ? my_row : m - 1;
-        const int my_pos = P0 + my_row_c;
-        const bool wave_active = wr0 < m;
-        const int wpos_min = P0 + (wave_active ? wr0 : m - 1);
-        const int wpos_max = P0 + min(wr0 + 31, m - 1);
+        const bool row_ok = my_row < n_rows;
+        const int my_row_c = row_ok ? my_row : n_rows - 1;
+        const int my_tok = tok_of(my_row_c);
+        const int my_h = SPLIT ? g * kv_mul + (my_row_c - my_tok * kv_mul) : h;
+        const int my_pos = P0 + my_tok;
+        const bool wave_active = wr0 < n_rows;
+        const int wpos_min = P0 + tok_of(wave_active ? wr0 : n_rows - 1);
+        const int wpos_max = P0 + tok_of(min(wr0 + 31, n_rows - 1));
         // Keys visible to the row at position pos: [row_lo(pos), row_hi(pos)].
         // Causal: [pos + 1 - W (or 0), pos].  Bidirectional image block (the m
         // rows are one block, LanguageAttentionPolicy::visible_keys,
@@ -369,14 +387,14 @@ __device__ __forceinline__ void prefill_body(const PrefillLaunch& p, const void*
         uint4 qf[D / 16];
         uint4 qfl[kSplit && !kQloLds ? D / 16 : 1];
         bool q_done = false;
-        if constexpr (D == 128) {
+        if constexpr (D == 128 && !SPLIT) {
             if (p.q_raw) {
                 pf_prepare_q<DT, D>(p, my_row_c, h, lg, qf, qfl);
                 q_done = true;
             }
         }
         if (!q_done) {
-            const size_t qoff = ((size_t)my_row_c * p.n_heads + h) * D + 8 * lg;
+            const size_t qoff = ((size_t)my_tok * p.n_heads + my_h) * D + 8 * lg;
             const uint16_t* qrow = (const uint16_t*)p.q + qoff;
 #pragma unroll
             for (int s = 0; s < D / 16; s++) qf[s] = *(const uint4*)(qrow + 16 * s);
@@ -413,10 +431,17 @@ __device__ __forceinline__ void prefill_body(const PrefillLaunch& p, const void*
         }
 
         // keys [kbeg, kend) of the cache are visible to some row of this block
-        const int kend = p.bidirectional ? P0 + m : P0 + min(q0 + BM, m);
-        const int kbeg = max(0, row_lo(P0 + q0));
-        const int t_first = kbeg / BN * BN;
-        const int n_tiles = (kend - t_first + BN - 1) / BN;
+        const int kend = pf_key_hi(P0, tok_of(min(q0 + BM, n_rows) - 1), m, p.bidirectional);
+        const int kbeg = max(0, row_lo(P0 + tok_of(q0)));
+        int t_first = kbeg / BN * BN;
+        int n_tiles = (kend - t_first + BN - 1) / BN;
+        if constexpr (SPLIT) {
+            // this workgroup's tiles of the block (the same count on every thread)
+            const int it0 = piece * p.split.ct;
+            if (it0 >= n_tiles) return;
+            n_tiles = min(n_tiles - it0, p.split.ct);
+            t_first += it0 * BN;
+        }
 
         // Issue the DMA of the tile starting at key t0.  Rows past kend - 1 are
         // clamped to it (they are masked; the clamp keeps P.V free of stale data).
@@ -660,6 +685,7 @@ __device__ __forceinline__ void prefill_body(const PrefillLaunch& p, const void*
                 const float m1 = mlb[lane], l1 = mlb[64 + lane];
                 const float mm = fmaxf(mrow, m1);
                 const float a0 = __builtin_amdgcn_exp2f(mrow - mm), a1 = __builtin_amdgcn_exp2f(m1 - mm);
+                mrow = mm;
                 lrow = lrow * a0 + l1 * a1;
 #pragma unroll
                 for (int dt = 0; dt < D / 32; dt++)
@@ -668,6 +694,21 @@ __device__ __forceinline__ void prefill_body(const PrefillLaunch& p, const void*
             }
         }
         const float lsum = pf_xsum32(lrow);
+        if constexpr (SPLIT) {
+            if (kh == 0 && wave_active) {
+                const size_t unit = ((size_t)(g * n_qb + qblk) * p.split.n_splits + piece) * RW + rw;
+                float4* po = (float4*)p.split.ws_o + unit * (D / 8) * 64;
+#pragma unroll
+                for (int dt = 0; dt < D / 32; dt++)
+#pragma unroll
+                    for (int jb = 0; jb < 4; jb++)
+                        po[(4 * dt + jb) * 64 + lane] = make_float4(o[dt][4 * jb + 0], o[dt][4 * jb + 1],
+                                                                    o[dt][4 * jb + 2], o[dt][4 * jb + 3]);
+                p.split.ws_ml[unit * 128 + lane] = mrow;
+                p.split.ws_ml[unit * 128 + 64 + lane] = lsum;
+            }
+            return;
+        }
         const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
         if (row_ok && kh == 0) {
             float* orow = p.out + ((size_t)my_row * p.n_heads + h) * D;
@@ -703,36 +744,160 @@ __device__ __forceinline__ void prefill_body(const PrefillLaunch& p, const void*
     __shared__ __attribute__((aligned(16))) uint16_t Vs1[PfTile<D, NW, KH>::BN * D];  \
     __shared__ __attribute__((aligned(16))) uint4 Qlo[(QLO) ? NW * (D / 16) * 64 : 1]
 
-template <typename DT, int D, int NW, int KH>
+template <typename DT, int D, int NW, int KH, bool SPLIT>
 __global__ __launch_bounds__(NW * 64, (PfTile<D, NW, KH>::kWaves)) void prefill_kernel(const PrefillLaunch p) {
     GR_PF_LDS(D, NW, KH, Mfma32<DT>::kSplit && D == 256);
-    prefill_body<DT, D, NW, KH>(p, p.k_cache, p.v_cache, p.cache_row_stride, 0, Ks0, Ks1, Vs0, Vs1, Qlo);
+    prefill_body<DT, D, NW, KH, SPLIT>(p, p.k_cache, p.v_cache, p.cache_row_stride, 0, Ks0, Ks1, Vs0, Vs1, Qlo);
 }
 
 // bf16 cache with an exact f16 copy of its visible rows: the single-pass f16
 // path on the copy, or, when the copy could not hold every value (the flag
 // carries this launch's epoch), the bf16 hi + lo path on the cache itself.
-template <int D, int NW, int KH>
+template <int D, int NW, int KH, bool SPLIT>
 __global__ __launch_bounds__(NW * 64, (PfTile<D, NW, KH>::kWaves)) void prefill_bf16x_kernel(const PrefillLaunch p) {
     GR_PF_LDS(D, NW, KH, D == 256);
     if (*p.f16_flag != p.f16_epoch)
-        prefill_body<F16, D, NW, KH>(p, p.k_f16, p.v_f16, p.f16_row_stride, p.f16_row0, Ks0, Ks1, Vs0, Vs1, Qlo);
+        prefill_body<F16, D, NW, KH, SPLIT>(p, p.k_f16, p.v_f16, p.f16_row_stride, p.f16_row0, Ks0, Ks1, Vs0, Vs1, Qlo);
     else
-        prefill_body<BF16, D, NW, KH>(p, p.k_cache, p.v_cache, p.cache_row_stride, 0, Ks0, Ks1, Vs0, Vs1, Qlo);
+        prefill_body<BF16, D, NW, KH, SPLIT>(p, p.k_cache, p.v_cache, p.cache_row_stride, 0, Ks0, Ks1, Vs0, Vs1, Qlo);
 }
 #undef GR_PF_LDS
 
-template <typename DT, int D, int NW, int KH = 1>
+// Merges the partials of a key-split launch.  Unit = 32 packed rows x 32 head
+// elements (one O^T accumulator tile) of one (KV head, query block, row group);
+// its pieces are taken by WPU waves in turn, four at a time (their loads in
+// flight together), and the waves' sums meet in LDS.
+template <int WPU>
+__global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillCombineLaunch p) {
+    __shared__ float part[WPU > 1 ? WPU - 1 : 1][18][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int ln = lane & 31, lg = lane >> 5;
+    const int kv_mul = p.n_heads / p.n_kv_heads;
+    const int ND = p.head_dim / 32, RW = p.split.bm / 32;
+    const int unit = WPU > 1 ? (int)blockIdx.x : (int)blockIdx.x * 4 + wave;
+    const int dt = unit % ND, rw = unit / ND % RW, gq = unit / ND / RW;
+    if (gq >= p.n_kv_heads * p.split.n_qb) return;
+    const int qb = gq % p.split.n_qb, g = gq / p.split.n_qb;
+    const int row = qb * p.split.bm + rw * 32 + ln;
+    if (qb * p.split.bm + rw * 32 >= p.n_tokens * kv_mul) return;  // uniform over the workgroup when WPU > 1
+    const int tiles = pf_split_tiles(qb, p.split.bm, p.split.bn, p.n_tokens, kv_mul, p.base_pos, p.window,
+                                     p.bidirectional);
+    const int ns = (tiles + p.split.ct - 1) / p.split.ct;
+    const size_t u0 = (size_t)gq * p.split.n_splits * RW + rw;
+    float M = -1e30f, L = 0.0f;
+    float o[16];
+#pragma unroll
+    for (int e = 0; e < 16; e++) o[e] = 0.0f;
+    for (int s0 = WPU > 1 ? wave : 0; s0 < ns; s0 += 4 * WPU) {
+        float mv[4], lv[4];
+        float4 ov[4][4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const size_t un = u0 + (size_t)min(s0 + u * WPU, ns - 1) * RW;
+            const bool in = s0 + u * WPU < ns;
+            const float mm = p.split.ws_ml[un * 128 + lane], ll = p.split.ws_ml[un * 128 + 64 + lane];
+            mv[u] = in ? mm : -1e30f;
+            lv[u] = in ? ll : 0.0f;
+            const float4* po = (const float4*)p.split.ws_o + un * ND * 256 + (size_t)dt * 256 + lane;
+#pragma unroll
+            for (int jb = 0; jb < 4; jb++) ov[u][jb] = po[jb * 64];
+        }
+        float mm = M;
+#pragma unroll
+        for (int u = 0; u < 4; u++) mm = fmaxf(mm, mv[u]);
+        const float a = __builtin_amdgcn_exp2f(M - mm);
+        M = mm;
+        L *= a;
+#pragma unroll
+        for (int e = 0; e < 16; e++) o[e] *= a;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (s0 + u * WPU >= ns) break;
+            const float w = __builtin_amdgcn_exp2f(mv[u] - mm);
+            L += lv[u] * w;
+#pragma unroll
+            for (int jb = 0; jb < 4; jb++) {
+                o[4 * jb + 0] += ov[u][jb].x * w;
+                o[4 * jb + 1] += ov[u][jb].y * w;
+                o[4 * jb + 2] += ov[u][jb].z * w;
+                o[4 * jb + 3] += ov[u][jb].w * w;
+            }
+        }
+    }
+    if constexpr (WPU > 1) {
+        if (wave > 0) {
+#pragma unroll
+            for (int e = 0; e < 16; e++) part[wave - 1][e][lane] = o[e];
+            part[wave - 1][16][lane] = M;
+            part[wave - 1][17][lane] = L;
+        }
+        __syncthreads();
+        if (wave > 0) return;
+        float mm = M;
+#pragma unroll
+        for (int w = 0; w < WPU - 1; w++) mm = fmaxf(mm, part[w][16][lane]);
+        const float a = __builtin_amdgcn_exp2f(M - mm);
+        L *= a;
+#pragma unroll
+        for (int e = 0; e < 16; e++) o[e] *= a;
+#pragma unroll
+        for (int w = 0; w < WPU - 1; w++) {
+            const float b = __builtin_amdgcn_exp2f(part[w][16][lane] - mm);
+            L += part[w][17][lane] * b;
+#pragma unroll
+            for (int e = 0; e < 16; e++) o[e] += part[w][e][lane] * b;
+        }
+    }
+    if (row >= p.n_tokens * kv_mul) return;
+    const int tok = row / kv_mul, h = g * kv_mul + row % kv_mul;
+    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    float* orow = p.out + ((size_t)tok * p.n_heads + h) * p.head_dim;
+    const float* gt = p.gate.at(tok, h);  // Qwen3.5 output gate, or null
+#pragma unroll
+    for (int jb = 0; jb < 4; jb++) {
+        const int d0 = 32 * dt + 8 * jb + 4 * lg;
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            v[e] = o[4 * jb + e] * inv;
+            if (gt) v[e] = gate_mul(v[e], gt[d0 + e]);
+        }
+        *(float4*)(orow + d0) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+}
+
+hipError_t launch_prefill_combine(const PrefillCombineLaunch& p, hipStream_t st) {
+    const int units = p.n_kv_heads * p.split.n_qb * (p.split.bm / 32) * (p.head_dim / 32);
+    if (p.split.n_splits > 4) prefill_combine_kernel<4><<<units, 256, 0, st>>>(p);
+    else prefill_combine_kernel<1><<<(units + 3) / 4, 256, 0, st>>>(p);
+    return hipGetLastError();
+}
+
+template <typename DT, int D, int NW, int KH = 1, bool SPLIT = false>
 static hipError_t launch_prefill_d(const PrefillLaunch& p, hipStream_t st) {
     constexpr int BM = NW / KH * 32;
     const int n_qb = (p.n_tokens + BM - 1) / BM;
-    const int n_items = p.n_heads * ((n_qb + 1) / 2);  // query blocks paired heavy + light
-    dim3 grid(8 * ((n_items + 7) / 8));
+    // query blocks paired heavy + light
+    const int n_items = p.n_heads * ((n_qb + 1) / 2);
+    const dim3 grid(SPLIT ? pf_split_grid(p.n_kv_heads, p.split.n_qb, p.split.n_splits) : 8 * ((n_items + 7) / 8));
     if (std::is_same<DT, BF16>::value && p.k_f16)
-        prefill_bf16x_kernel<D, NW, KH><<<grid, NW * 64, 0, st>>>(p);
+        prefill_bf16x_kernel<D, NW, KH, SPLIT><<<grid, NW * 64, 0, st>>>(p);
     else
-        prefill_kernel<DT, D, NW, KH><<<grid, NW * 64, 0, st>>>(p);
-    return hipGetLastError();
+        prefill_kernel<DT, D, NW, KH, SPLIT><<<grid, NW * 64, 0, st>>>(p);
+    hipError_t e = hipGetLastError();
+    if (!SPLIT || e != hipSuccess) return e;
+    PrefillCombineLaunch c{};
+    c.n_tokens = p.n_tokens;
+    c.n_heads = p.n_heads;
+    c.n_kv_heads = p.n_kv_heads;
+    c.head_dim = D;
+    c.base_pos = (int)p.base_pos;
+    c.window = p.window;
+    c.bidirectional = p.bidirectional;
+    c.split = p.split;
+    c.out = p.out;
+    c.gate = p.gate;
+    return launch_prefill_combine(c, st);
 }
 
 // Workgroup shape (d <= 128): eight waves of 256 rows once those workgroups
@@ -742,16 +907,66 @@ static hipError_t launch_prefill_d(const PrefillLaunch& p, hipStream_t st) {
 // workgroups) 44.0 -> 36.4 us per call; at d128 (32 / 8 heads, S = 2048, 256
 // workgroups) the key halves were 1.5% slower than four waves.
 enum { kPfWaves8 = 8, kPfWaves4 = 4, kPfKeyHalves = 2 };
+constexpr int kPfCUs = 256;
 static int prefill_pick(const PrefillLaunch& p) {
-    constexpr int kCUs = 256;
     if (p.head_dim > 128) return kPfWaves4;
     const int n_qb8 = (p.n_tokens + 255) / 256, n_qb4 = (p.n_tokens + 127) / 128;
-    if (p.n_heads * ((n_qb8 + 1) / 2) >= kCUs) return kPfWaves8;
-    return p.head_dim == 64 && p.n_heads * ((n_qb4 + 1) / 2) <= kCUs ? kPfKeyHalves : kPfWaves4;
+    if (p.n_heads * ((n_qb8 + 1) / 2) >= kPfCUs) return kPfWaves8;
+    return p.head_dim == 64 && p.n_heads * ((n_qb4 + 1) / 2) <= kPfCUs ? kPfKeyHalves : kPfWaves4;
+}
+
+// Resident workgroups of the split kernels (two per CU at d <= 128, one at 256),
+// and the rows and keys of their tiles.
+struct PfSplitShape {
+    int slots, bm, bn;
+};
+static PfSplitShape pf_split_shape(int head_dim) {
+    if (head_dim == 64) return {2 * kPfCUs, 128, PfTile<64, 8, 2>::BN};
+    if (head_dim == 128) return {2 * kPfCUs, 128, PfTile<128, 4>::BN};
+    return {kPfCUs, 128, PfTile<256, 4>::BN};
+}
+
+// Split or not: in tiles of 128 rows x BN keys, the unsplit launch takes its longest
+// pair of blocks (it has at most one workgroup per CU here); the split one at least
+// one piece and its share of all tiles, 1.1 for the uneven finish, a tile for the
+// combine launch and 0.03 (d128) per workgroup for its partials.  Fitted to 74
+// launches, 16 to 4096 tokens after 0 to 8000, five head shapes: the rule takes
+// the slower side by at most 4%.  MI355X, us per call (prep included), unsplit ->
+// split: 32 / 8 heads d128, 64 tokens after 4000 78.5 -> 29, 512 after 8000 302 -> 92,
+// 1500 after 8000 325 -> 267; 14 / 2 heads d64, 203 after 4000 83 -> 25, 1500 after
+// 8000 167 -> 80; 8 / 4 heads d256, 512 after 8000 543 -> 61.  Not split: 1500 tokens
+// from 0, d128 54 (63 split); 4096 from 0, d64 58 (73 split).
+PrefillSplit prefill_split_plan(int n_tokens, int n_heads, int n_kv_heads, int head_dim, int base_pos, int window,
+                                int bidirectional) {
+    const PfSplitShape sh = pf_split_shape(head_dim);
+    if (n_tokens <= 0) return {};
+    const int n_qb = (n_tokens - 1) / sh.bm + 1;
+    if ((int64_t)n_heads * ((n_qb + 1) / 2) > kPfCUs) return {};
+    const PrefillSplit s = pf_split_plan(n_tokens, n_heads, n_kv_heads, base_pos, window, bidirectional, sh.bm, sh.bn,
+                                         sh.slots, 128 / sh.bn);
+    if (s.n_splits == 0) return s;
+    auto block = [&](int qb) {
+        return pf_split_tiles(qb, sh.bm, sh.bn, n_tokens, 1, base_pos, window, bidirectional);
+    };
+    const float whole = (float)(block(n_qb - 1) + (n_qb > 1 ? block(0) : 0));
+    const float share = (float)s.tiles / kPfCUs;
+    const float cost = 1.1f * (share > s.ct ? share : (float)s.ct) + 1.0f + 0.03f * s.wgs * head_dim / 128;
+    return cost < whole ? s : PrefillSplit{};
+}
+
+size_t prefill_split_ws_bytes(int head_dim) {
+    const PfSplitShape sh = pf_split_shape(head_dim);
+    return pf_split_ws_bytes(sh.slots, sh.bm, head_dim);
 }
 
 template <typename DT>
 static hipError_t launch_prefill_dt(const PrefillLaunch& p, hipStream_t st) {
+    if (p.split.n_splits > 0) switch (p.head_dim) {
+            case 64: return launch_prefill_d<DT, 64, 8, 2, true>(p, st);
+            case 128: return launch_prefill_d<DT, 128, 4, 1, true>(p, st);
+            case 256: return launch_prefill_d<DT, 256, 4, 1, true>(p, st);
+            default: return hipErrorInvalidValue;
+        }
     switch (p.head_dim) {
         case 64:
             switch (prefill_pick(p)) {

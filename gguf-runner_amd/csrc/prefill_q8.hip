@@ -4,6 +4,8 @@
 // token-serial attention of the prefill loop (inference.rs:2981-3017, one
 // attention_token per token) for Q8 run states: one launch per chunk, every
 // K / V tile read once per 128 (d64, d128) or 64 (d256) query rows.
+// Short chunks over long caches launch too few such workgroups: they pack the query
+// heads of a KV head into the rows and are cut along the keys (prefill_split.hpp).
 //
 // Workgroup = row groups of 32 query rows of one query head x 2 key halves,
 // wave (row group, half) taking the 32-key sub-tiles 2 j + half of every tile;
@@ -109,7 +111,8 @@ __device__ __forceinline__ int q8p_swz(int r) {
     else return ((r << 2) ^ (r << 1) ^ (r >> 2)) & 15;
 }
 
-template <int D, bool BLOCK>
+// SPLIT: one piece of the keys of a block of packed rows (prefill_split.hpp).
+template <int D, bool BLOCK, bool SPLIT>
 __global__ __launch_bounds__(Q8Tile<D>::NT, 1) void prefill_q8_kernel(const PrefillQ8Launch p) {
     constexpr int KH = Q8Tile<D>::KH, RG = Q8Tile<D>::RG;
     constexpr int NT = Q8Tile<D>::NT;     // threads
@@ -143,11 +146,19 @@ __global__ __launch_bounds__(Q8Tile<D>::NT, 1) void prefill_q8_kernel(const Pref
     const int m = p.n_tokens;
     const int P0 = (int)p.base_pos;
     const int W = p.window;
-    const int n_qb = (m + BM - 1) / BM;
-    const int h = blockIdx.x;
-    const int qblk = n_qb - 1 - (int)blockIdx.y;  // the longest query blocks first
     const int kv_mul = p.n_heads / p.n_kv_heads;
-    const int g = h / kv_mul;
+    const int n_rows = SPLIT ? m * kv_mul : m;
+    const int n_qb = (n_rows + BM - 1) / BM;
+    // token of a row (rows are packed (token, query head of the group) when SPLIT)
+    auto tok_of = [&](int r) { return SPLIT ? r / kv_mul : r; };
+    PfSplitItem si{0, 0, 0};
+    if constexpr (SPLIT) {
+        si = pf_split_item((int)blockIdx.x, p.n_kv_heads, p.split.n_qb, p.split.n_splits);
+        if (si.qb >= n_qb) return;
+    }
+    const int h = SPLIT ? 0 : blockIdx.x;
+    const int qblk = SPLIT ? si.qb : n_qb - 1 - (int)blockIdx.y;  // the longest query blocks first
+    const int g = SPLIT ? si.g : h / kv_mul;
     const int8_t* kc = p.k_codes + (size_t)g * D;
     const int8_t* vc = p.v_codes + (size_t)g * D;
     const int64_t rs = p.row_stride;
@@ -156,14 +167,28 @@ __global__ __launch_bounds__(Q8Tile<D>::NT, 1) void prefill_q8_kernel(const Pref
     const int64_t srs = p.scale_row_stride;
 
     const int q0 = qblk * BM;
+    // keys [kbeg, kend) are visible to some row of this block
+    const int kend = pf_key_hi(P0, tok_of(min(q0 + BM, n_rows) - 1), m, p.bidirectional);
+    const int kbeg = pf_key_lo(P0, tok_of(q0), W, p.bidirectional);
+    int t_first = kbeg / BN * BN;
+    int n_tiles = (kend - t_first + BN - 1) / BN;
+    if constexpr (SPLIT) {
+        // this workgroup's tiles of the block (the same count on every thread)
+        const int it0 = si.piece * p.split.ct;
+        if (it0 >= n_tiles) return;
+        n_tiles = min(n_tiles - it0, p.split.ct);
+        t_first += it0 * BN;
+    }
     const int wr0 = q0 + rg * 32;
     const int my_row = wr0 + ln;
-    const bool row_ok = my_row < m;
-    const int my_row_c = row_ok ? my_row : m - 1;
-    const int my_pos = P0 + my_row_c;
-    const bool wave_active = wr0 < m;
-    const int wpos_min = P0 + (wave_active ? wr0 : m - 1);
-    const int wpos_max = P0 + min(wr0 + 31, m - 1);
+    const bool row_ok = my_row < n_rows;
+    const int my_row_c = row_ok ? my_row : n_rows - 1;
+    const int my_tok = tok_of(my_row_c);
+    const int my_h = SPLIT ? g * kv_mul + (my_row_c - my_tok * kv_mul) : h;
+    const int my_pos = P0 + my_tok;
+    const bool wave_active = wr0 < n_rows;
+    const int wpos_min = P0 + tok_of(wave_active ? wr0 : n_rows - 1);
+    const int wpos_max = P0 + tok_of(min(wr0 + 31, n_rows - 1));
     // Keys visible to the row at position pos: [row_lo(pos), row_hi(pos)]; causal
     // [pos + 1 - W (or 0), pos], image block [min(pos + 1 - W (or 0), P0), P0 + m - 1]
     // (LanguageAttentionPolicy::visible_keys, attention.rs:74-96).
@@ -180,7 +205,7 @@ __global__ __launch_bounds__(Q8Tile<D>::NT, 1) void prefill_q8_kernel(const Pref
     uint4 qf[D / 16], qfl[kQloLds ? 1 : D / 16];
     float qfac;
     {
-        const float* qrow = p.q + ((size_t)my_row_c * p.n_heads + h) * D + 8 * lg;
+        const float* qrow = p.q + ((size_t)my_tok * p.n_heads + my_h) * D + 8 * lg;
         const float qs = p.score_scale * 1.44269504088896340736f;
         float qv[D / 16][8];
         float amax = 0.0f;
@@ -216,12 +241,6 @@ __global__ __launch_bounds__(Q8Tile<D>::NT, 1) void prefill_q8_kernel(const Pref
         if constexpr (kQloLds) return Qlo[(rg * (D / 16) + s) * 64 + lane];
         else return qfl[s];
     };
-
-    // keys [kbeg, kend) are visible to some row of this block
-    const int kend = p.bidirectional ? P0 + m : P0 + min(q0 + BM, m);
-    const int kbeg = max(0, row_lo(P0 + q0));
-    const int t_first = kbeg / BN * BN;
-    const int n_tiles = (kend - t_first + BN - 1) / BN;
 
     // Tile staging registers; rows past kend - 1 are clamped to it (masked).
     uint4 kreg[KCH], vreg[KCH];
@@ -461,6 +480,7 @@ __global__ __launch_bounds__(Q8Tile<D>::NT, 1) void prefill_q8_kernel(const Pref
         const float lb = Ms[(rg * (2 + NBS) + 1) * 64 + lane];
         const float mm = fmaxf(mrow, mb);
         const float aa = __builtin_amdgcn_exp2f(mrow - mm), ab = __builtin_amdgcn_exp2f(mb - mm);
+        mrow = mm;
         lrow = lrow * aa + lb * ab;
 #pragma unroll
         for (int b = 0; b < NBS; b++) {
@@ -482,6 +502,21 @@ __global__ __launch_bounds__(Q8Tile<D>::NT, 1) void prefill_q8_kernel(const Pref
     }
 
     const float lsum = q8p_xsum32(lrow);
+    if constexpr (SPLIT) {
+        static_assert(KH == 2, "the merged O carries no 1 / pw factor");
+        if (!wave_active) return;
+        const size_t unit = ((size_t)(g * n_qb + qblk) * p.split.n_splits + si.piece) * RG + rg;
+        float4* po = (float4*)p.split.ws_o + unit * (D / 8) * 64;
+#pragma unroll
+        for (int dt = 0; dt < NB; dt++)
+#pragma unroll
+            for (int jb = 0; jb < 4; jb++)
+                po[(4 * dt + jb) * 64 + lane] =
+                    make_float4(o[dt][4 * jb + 0], o[dt][4 * jb + 1], o[dt][4 * jb + 2], o[dt][4 * jb + 3]);
+        p.split.ws_ml[unit * 128 + lane] = mrow;
+        p.split.ws_ml[unit * 128 + 64 + lane] = lsum;
+        return;
+    }
     if (row_ok) {
         float* orow = p.out + ((size_t)my_row * p.n_heads + h) * D;
         const float* gt = p.gate.at(my_row, h);  // Qwen3.5 output gate, or null
@@ -511,12 +546,62 @@ __global__ __launch_bounds__(Q8Tile<D>::NT, 1) void prefill_q8_kernel(const Pref
 
 template <int D, bool BLOCK>
 hipError_t launch_q8_d(const PrefillQ8Launch& p, hipStream_t st) {
+    if (p.split.n_splits > 0) {
+        const int grid = pf_split_grid(p.n_kv_heads, p.split.n_qb, p.split.n_splits);
+        prefill_q8_kernel<D, BLOCK, true><<<grid, Q8Tile<D>::NT, 0, st>>>(p);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        PrefillCombineLaunch c{};
+        c.n_tokens = p.n_tokens;
+        c.n_heads = p.n_heads;
+        c.n_kv_heads = p.n_kv_heads;
+        c.head_dim = D;
+        c.base_pos = (int)p.base_pos;
+        c.window = p.window;
+        c.bidirectional = p.bidirectional;
+        c.split = p.split;
+        c.out = p.out;
+        c.gate = p.gate;
+        return launch_prefill_combine(c, st);
+    }
     const int n_qb = (p.n_tokens + Q8Tile<D>::BM - 1) / Q8Tile<D>::BM;
-    prefill_q8_kernel<D, BLOCK><<<dim3(p.n_heads, n_qb), Q8Tile<D>::NT, 0, st>>>(p);
+    prefill_q8_kernel<D, BLOCK, false><<<dim3(p.n_heads, n_qb), Q8Tile<D>::NT, 0, st>>>(p);
     return hipGetLastError();
 }
 
+constexpr int kQ8CUs = 256;  // resident workgroups: one per CU
+
+// Split or not, as prefill_split_plan's rule (tiles of BM rows x BN keys; the unsplit
+// launch, at most one workgroup per CU, takes its longest block).  MI355X, us of
+// gr_prefill_attention_chunk with its host rows, unsplit -> split: 32 / 8 heads
+// d128, 2 tokens after 4000 136 -> 42, 64 after 4000 285 -> 191, 512 after 4000 739 ->
+// 691; 14 / 2 heads d64, 64 after 4000 122 -> 59; 8 / 4 heads d256, 64 after 4000 297
+// -> 116.  Not split: chunks of 30 or fewer keys of history (equal within 3%).
+template <int D>
+PrefillSplit q8_plan(int n_tokens, int n_heads, int n_kv_heads, int base_pos, int window, int bidirectional) {
+    constexpr int BM = Q8Tile<D>::BM, BN = Q8Tile<D>::BN;
+    if (n_tokens <= 0) return {};
+    const int n_qb = (n_tokens - 1) / BM + 1;
+    if ((int64_t)n_heads * n_qb > kQ8CUs) return {};
+    const PrefillSplit s = pf_split_plan(n_tokens, n_heads, n_kv_heads, base_pos, window, bidirectional, BM, BN, kQ8CUs, 1);
+    if (s.n_splits == 0) return s;
+    const float whole = (float)pf_split_tiles(n_qb - 1, BM, BN, n_tokens, 1, base_pos, window, bidirectional);
+    const float share = (float)s.tiles / kQ8CUs;
+    const float cost = 1.1f * (share > s.ct ? share : (float)s.ct) + 1.0f + 0.015f * s.wgs * D / 128;
+    return cost < whole ? s : PrefillSplit{};
+}
+
 }  // namespace
+
+PrefillSplit prefill_q8_split_plan(int n_tokens, int n_heads, int n_kv_heads, int head_dim, int base_pos, int window,
+                                   int bidirectional) {
+    switch (head_dim) {
+        case 64: return q8_plan<64>(n_tokens, n_heads, n_kv_heads, base_pos, window, bidirectional);
+        case 128: return q8_plan<128>(n_tokens, n_heads, n_kv_heads, base_pos, window, bidirectional);
+        case 256: return q8_plan<256>(n_tokens, n_heads, n_kv_heads, base_pos, window, bidirectional);
+        default: return {};
+    }
+}
 
 hipError_t launch_prefill_q8(const PrefillQ8Launch& p, hipStream_t st) {
     if (p.n_tokens <= 0) return hipSuccess;

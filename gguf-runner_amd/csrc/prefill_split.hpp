@@ -1,0 +1,122 @@
+// Key-split prefill launches (short chunks over long caches): the plan, shared by
+// the host and the kernels.
+//
+// A launch whose (query head, query block) workgroups leave most CUs idle is cut
+// along the keys instead.  The kv_mul query heads of a KV head are packed into
+// the rows of a query block (row r of KV head g is token r / kv_mul, query head
+// g * kv_mul + r % kv_mul: a 16-token chunk fills its 32-row waves, and a K / V
+// tile is read once for the whole group), and every block's range of BN-key tiles
+// is cut into pieces of `ct` tiles, one workgroup each.  A workgroup writes its
+// unnormalised f32 O^T accumulators and each row's (maximum, sum) as partials,
+// in the register layout of the MFMA accumulators; the combine kernel merges them.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace gr {
+
+struct PrefillSplit {
+    int n_splits = 0;        // pieces of the longest block; 0: not split
+    int ct = 0;              // tiles per piece
+    int n_qb = 0;            // query blocks per KV head
+    int bm = 0, bn = 0;      // rows per block, keys per tile
+    int64_t tiles = 0;       // tiles of all blocks
+    int wgs = 0;             // workgroups with tiles
+    float* ws_o = nullptr;   // [g][query block][piece][row group of 32][d / 32][4][lane][4]
+    float* ws_ml = nullptr;  // [g][query block][piece][row group of 32][m | l][lane]
+};
+
+// Keys [lo, hi) that the tokens tok0 .. tok1 of a chunk see (hi exclusive).
+__host__ __device__ inline int pf_key_lo(int p0, int tok0, int window, int bidirectional) {
+    int lo = window > 0 ? p0 + tok0 + 1 - window : 0;
+    if (bidirectional && lo > p0) lo = p0;
+    return lo > 0 ? lo : 0;
+}
+__host__ __device__ inline int pf_key_hi(int p0, int tok1, int n_tokens, int bidirectional) {
+    return bidirectional ? p0 + n_tokens : p0 + tok1 + 1;
+}
+
+// Tiles of query block qb of a split launch.
+__host__ __device__ inline int pf_split_tiles(int qb, int bm, int bn, int n_tokens, int kv_mul, int p0, int window,
+                                              int bidirectional) {
+    const int rows = n_tokens * kv_mul;
+    const int last = (qb + 1) * bm < rows ? (qb + 1) * bm - 1 : rows - 1;
+    const int first = pf_key_lo(p0, qb * bm / kv_mul, window, bidirectional) / bn * bn;
+    return (pf_key_hi(p0, last / kv_mul, n_tokens, bidirectional) - first + bn - 1) / bn;
+}
+
+// Workgroup b of a split launch.  It runs on XCD b % 8, and the XCDs share the KV
+// heads: one XCD takes n_kv / 8 heads, or 8 / n_kv XCDs take the query blocks of one
+// head in turn (so that a head's tiles stay in few L2s and the short and the long
+// blocks of a first chunk spread evenly); other head counts go round the XCDs item
+// by item.  qb may come out past the last block: an idle workgroup.
+struct PfSplitItem {
+    int g, piece, qb;
+};
+__host__ __device__ inline int pf_split_xcds(int n_kv) { return n_kv % 8 == 0 ? 1 : (8 % n_kv == 0 ? 8 / n_kv : 0); }
+__host__ __device__ inline int pf_split_grid(int n_kv, int n_qb, int n_splits) {
+    const int r = pf_split_xcds(n_kv);
+    if (r == 0) return n_kv * n_qb * n_splits;
+    return 8 * ((n_kv * r + 7) / 8) * ((n_qb + r - 1) / r) * n_splits;
+}
+__host__ __device__ inline PfSplitItem pf_split_item(int b, int n_kv, int n_qb, int n_splits) {
+    const int r = pf_split_xcds(n_kv);
+    if (r == 0) return {b / (n_qb * n_splits), b / n_qb % n_splits, b % n_qb};
+    const int per = (n_qb + r - 1) / r;  // blocks of a head on one XCD
+    const int x = b & 7, i = b >> 3;
+    return {x / r + i / (per * n_splits) * 8, i / per % n_splits, i % per * r + x % r};
+}
+
+// Partial slots (workgroups) a split launch may have, for `slots` resident
+// workgroups: causal blocks of a first chunk are half empty in the
+// [block][piece] index, so twice the resident number.
+constexpr int kPfSplitSlots = 2;
+constexpr size_t pf_split_ws_bytes(int slots, int bm, int head_dim) {
+    return (size_t)kPfSplitSlots * slots * bm * (head_dim + 4) * 4;
+}
+
+// Bytes of a plan's partials, and their carving: ws_ml, then ws_o.
+inline size_t pf_split_part_bytes(const PrefillSplit& s, int n_kv, int head_dim) {
+    return (size_t)s.n_qb * n_kv * s.n_splits * s.bm * (head_dim + 4) * 4;
+}
+inline void pf_split_carve(PrefillSplit& s, int n_kv, void* ws) {
+    s.ws_ml = (float*)ws;
+    s.ws_o = s.ws_ml + (size_t)s.n_qb * n_kv * s.n_splits * s.bm * 4;
+}
+
+// The smallest piece of at least min_ct tiles whose workgroups all fit the
+// `slots` the GPU holds at once (0 splits if there is none worth having: pieces
+// as long as the blocks).
+inline PrefillSplit pf_split_plan(int n_tokens, int n_heads, int n_kv, int p0, int window, int bidirectional, int bm,
+                                  int bn, int slots, int min_ct) {
+    PrefillSplit s;
+    const int kv_mul = n_heads / n_kv;
+    s.bm = bm, s.bn = bn;
+    s.n_qb = (int)(((int64_t)n_tokens * kv_mul + bm - 1) / bm);
+    auto tiles = [&](int qb) { return pf_split_tiles(qb, bm, bn, n_tokens, kv_mul, p0, window, bidirectional); };
+    int longest = 0;
+    int64_t total = 0;
+    for (int qb = 0; qb < s.n_qb; qb++) {
+        const int t = tiles(qb);
+        longest = t > longest ? t : longest;
+        total += t;
+    }
+    int ct = (int)((total * n_kv + slots - 1) / slots);
+    if (ct < min_ct) ct = min_ct;
+    for (; ct < longest; ct++) {
+        int64_t wgs = 0;
+        for (int qb = 0; qb < s.n_qb; qb++) wgs += (tiles(qb) + ct - 1) / ct;
+        const int n = (longest + ct - 1) / ct;
+        if (wgs * n_kv <= slots && (int64_t)s.n_qb * n_kv * n <= kPfSplitSlots * (int64_t)slots) {
+            s.ct = ct;
+            s.tiles = total * n_kv;
+            s.wgs = (int)(wgs * n_kv);
+            s.n_splits = n;
+            return s;
+        }
+    }
+    return s;
+}
+
+}  // namespace gr
