@@ -171,6 +171,22 @@ constexpr int kTpGl = kTpScale + 4 * kChunk * 4;
 constexpr int kTpBytes = 22 * 1024;  // 22 DMA rounds of 1 KB
 static_assert(kTpGl + 8 <= kTpBytes, "block layout");
 
+// bf16 rows: T as MFMA operands in lane order instead (16 bytes per lane, 1 KB each),
+// which the scan loads straight into registers.  Wave w of the scan owns tokens
+// tok(w, m) = 32 (w / 2) + 8 (m / 4) + 4 (w % 2) + m % 4, m < 16, so that the four
+// results of a lane group g are half of the eight consecutive reduction slots
+// 8 g .. 8 g + 7 of a k-step of 32 tokens.  Six (w, k-step) operands (w < 2: k-step
+// 0; w >= 2: 0 and 1) as three exact bf16 pieces each (hi, mid, lo by truncation),
+// [operand][piece][lane]: row tok(w, l % 16), columns 32 ks + 8 (l / 16) ..; then P
+// and the rest as above.
+constexpr int kBfT = 0;
+constexpr int kBfP = kBfT + 18 * 1024;
+constexpr int kBfScale = kBfP + kTpTiles * 1024;
+constexpr int kBfGl = kBfScale + 4 * kChunk * 4;
+constexpr int kBfBytes = 30 * 1024;
+static_assert(kBfGl + 8 <= kBfBytes, "block layout");
+__device__ __forceinline__ int bf_tok(int w, int m) { return 32 * (w >> 1) + 8 * (m >> 2) + 4 * (w & 1) + (m & 3); }
+
 // Workspace: [H][kScanBlocks] i32 chunks completed by each scan block (256-byte
 // aligned), then the (chunk, head) blocks.
 __host__ __device__ constexpr size_t dn_ws_head(int H) { return ((size_t)H * kScanBlocks * 4 + 255) / 256 * 256; }
@@ -243,9 +259,10 @@ __device__ __forceinline__ void dn_split3x4(const float* x, uint2* out) {
     uint32_t h[4], m[4], l[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) dn_split3(x[i], h[i], m[i], l[i]);
-    out[0] = make_uint2((h[0] >> 16) | h[1], (h[2] >> 16) | h[3]);
-    out[1] = make_uint2((m[0] >> 16) | m[1], (m[2] >> 16) | m[3]);
-    out[2] = make_uint2((l[0] >> 16) | l[1], (l[2] >> 16) | l[3]);
+    // one v_perm each: the upper halves of two words
+    out[0] = make_uint2(__builtin_amdgcn_perm(h[1], h[0], 0x07060302u), __builtin_amdgcn_perm(h[3], h[2], 0x07060302u));
+    out[1] = make_uint2(__builtin_amdgcn_perm(m[1], m[0], 0x07060302u), __builtin_amdgcn_perm(m[3], m[2], 0x07060302u));
+    out[2] = make_uint2(__builtin_amdgcn_perm(l[1], l[0], 0x07060302u), __builtin_amdgcn_perm(l[3], l[2], 0x07060302u));
 }
 
 template <int DT>
@@ -262,6 +279,7 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
     constexpr int D = 128;
     constexpr int C = kChunk;
     constexpr bool RAW = DT != GR_DTYPE_F32;  // 16-bit rows, Gram products on 16-bit MFMA
+    constexpr bool BF = DT == GR_DTYPE_BF16;  // operands for the bf16 scan
     constexpr int RS = D + 4;   // f32 row stride (floats): rows 4 banks apart
     constexpr int RS16 = D + 8; // 16-bit row stride (elements)
     constexpr int AMS = C + 4;  // A row stride
@@ -283,7 +301,7 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
     const int c = blockIdx.x, h = blockIdx.y, H = p.n_heads;
     const int t0 = c * C;
     const int Cn = min(C, p.n_tokens - t0);
-    char* blk = (char*)p.ws + dn_ws_head(H) + ((size_t)c * H + h) * kTpBytes;
+    char* blk = (char*)p.ws + dn_ws_head(H) + ((size_t)c * H + h) * (BF ? kBfBytes : kTpBytes);
     if (tid == 0) bad = 0;
     __syncthreads();
 
@@ -423,7 +441,7 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
                 const float pr = RAW ? qi[t] * ki[s] * acc[u][i] : acc[u][i];
                 const float v = s <= t ? dec * pr : 0.0f;
                 if (!is_finite_f(v)) bad = 1;
-                *(float*)(blk + kTpP + tt * 1024 + 4 * tp_elem(tl, l16)) = v;
+                *(float*)(blk + (BF ? kBfP : kTpP) + tt * 1024 + 4 * tp_elem(tl, l16)) = v;
             }
         }
     }
@@ -457,21 +475,41 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
             const int xi = (t >> 4) * 4 + (t & 3);
             x[xi] = ((t >> 2) & 3) == part ? val : x[xi];
         }
+        if constexpr (BF) __syncthreads();  // every read of A is done: T goes over it
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            if (u < wave) continue;  // T[s][col] = 0 above the diagonal tiles
+            if (!BF && u < wave) continue;  // T[s][col] = 0 above the diagonal tiles
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 const float v = x[4 * u + e];
                 if (!is_finite_f(v)) bad = 1;
-                *(float*)(blk + kTpT + tp_tri(u, wave) * 1024 + 4 * tp_elem(4 * part + e, lane >> 2)) = v;
+                if constexpr (BF) am[(16 * u + 4 * part + e) * AMS + col] = v;
+                else *(float*)(blk + kTpT + tp_tri(u, wave) * 1024 + 4 * tp_elem(4 * part + e, lane >> 2)) = v;
             }
+        }
+    }
+    if constexpr (BF) {
+        __syncthreads();
+        // T as operand pieces: wave w takes operands w and w + 4
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int op = wave + 4 * u;
+            if (op >= 6) break;
+            const int w = op < 2 ? op : (op + 2) >> 1, ks = op < 2 ? 0 : op & 1;
+            const float* src = am + bf_tok(w, l16) * AMS + 32 * ks + 8 * g;
+            uint2 lo[3], hi[3];
+            dn_split3x4(src, lo);
+            dn_split3x4(src + 4, hi);
+#pragma unroll
+            for (int pc = 0; pc < 3; pc++)
+                *(uint4*)(blk + kBfT + ((3 * op + pc) * 64 + lane) * 16) =
+                    make_uint4(lo[pc].x, lo[pc].y, hi[pc].x, hi[pc].y);
         }
     }
     // 4. row scales, gamma_last, flag
     if (tid < C) {
         const int t = tid;
-        float* sc = (float*)(blk + kTpScale);
+        float* sc = (float*)(blk + (BF ? kBfScale : kTpScale));
         const float v0 = bt[t], v1 = bt[t] * gm[t] * ki[t], v2 = gm[t] * qi[t], v3 = kf[t] * ki[t];
         sc[t] = v0;
         sc[C + t] = v1;
@@ -481,11 +519,11 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
         if (t == C - 1) {
             const float gl = gm[C - 1];
             if (!is_finite_f(gl)) bad = 1;
-            *(float*)(blk + kTpGl) = gl;
+            *(float*)(blk + (BF ? kBfGl : kTpGl)) = gl;
         }
     }
     __syncthreads();
-    if (tid == 0) *(int*)(blk + kTpGl + 4) = bad;
+    if (tid == 0) *(int*)(blk + (BF ? kBfGl : kTpGl) + 4) = bad;
 }
 
 // Raw buffer access: a buffer descriptor (base, stride 0, num_records = `bytes`:
@@ -601,15 +639,6 @@ __global__ __launch_bounds__(kChunkThreads, 1) void deltanet_chunk_scan_kernel(c
     __shared__ __attribute__((aligned(16))) float Sl[D * NC];
     __shared__ __attribute__((aligned(16))) float Xl[C * NC];
     __shared__ __attribute__((aligned(16))) float Dl[C * NC];
-    // bf16 rows (raw k / q exact as bf16): the K S0, Q S0 and state-update products
-    // run on v_mfma_f32_16x16x32_bf16 with the f32 operand as three exact bf16
-    // pieces (hi + mid + lo, three MFMAs), a third of the matrix-core time of the
-    // f32 MFMA.  The pieces in B-operand order: Sp[piece][k-step q][lane 16 g + n]
-    // = state rows 32 q + 8 g .. + 7 of column n; Dp the same for the scaled Delta
-    // rows (tokens).
-    constexpr bool BF = DT == GR_DTYPE_BF16;
-    __shared__ __attribute__((aligned(16))) uint4 Sp[BF ? 3 * (D / 32) * 64 : 1];
-    __shared__ __attribute__((aligned(16))) uint4 Dp[BF ? 3 * (C / 32) * 64 : 1];
     __shared__ int flag;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int l16 = lane & 15, g = lane >> 4;
@@ -628,31 +657,6 @@ __global__ __launch_bounds__(kChunkThreads, 1) void deltanet_chunk_scan_kernel(c
         Sl[e] = Sh[(size_t)(16 * q + 4 * gg + i) * D + c0 + n];
     }
     if (tid == 0) flag = 0;
-    // this wave's state rows 32 w + 16 tt + 4 g + (0..3) (an MFMA result's rows) as
-    // bf16 pieces: k-step w, lane 16 (2 tt + g / 2) + n, slots 4 (g % 2) ..
-    auto store_state_pieces = [&](const float* v0, const float* v1) {
-        if constexpr (BF) {
-#pragma unroll
-            for (int tt = 0; tt < 2; tt++) {
-                uint2 pcs[3];
-                dn_split3x4(tt ? v1 : v0, pcs);
-#pragma unroll
-                for (int pc = 0; pc < 3; pc++)
-                    *(uint2*)((char*)&Sp[(pc * (D / 32) + wave) * 64 + 16 * (2 * tt + (g >> 1)) + l16] + 8 * (g & 1)) =
-                        pcs[pc];
-            }
-        }
-    };
-    if constexpr (BF) {
-        __syncthreads();  // Sl complete
-        float v0[4], v1[4];
-        const float4 a = *(const float4*)(Sl + ((2 * wave) * 64 + lane) * 4);
-        const float4 b = *(const float4*)(Sl + ((2 * wave + 1) * 64 + lane) * 4);
-        v0[0] = a.x, v0[1] = a.y, v0[2] = a.z, v0[3] = a.w;
-        v1[0] = b.x, v1[1] = b.y, v1[2] = b.z, v1[3] = b.w;
-        store_state_pieces(v0, v1);
-    }
-
     // DMA round k of this wave for a K / Q tile: round I = wave + 4 k (1 KB) fills
     // position l % PPR of row I * RPK + l / PPR (lane l) with the piece that
     // belongs there (piece p of row t at position p ^ (t % 16))
@@ -755,30 +759,7 @@ __global__ __launch_bounds__(kChunkThreads, 1) void deltanet_chunk_scan_kernel(c
         // b: K S0, Q S0 for rows 16 w + (0..15); four chains (K / Q x even / odd i);
         //    the next chunk's K (and 16-bit Q) rounds between the MFMAs
         dn_f32x4 ak0 = {0.0f, 0.0f, 0.0f, 0.0f}, ak1 = ak0, aq0 = ak0, aq1 = ak0;
-        if constexpr (BF) {
-            // bf16: A = the raw row piece (k-step q: dims 32 q + 8 g .. + 7), B = the
-            // state's three pieces; ak1 / aq1 stay zero
-            const dn_i32x4 rk = rows_rsrc(p.k, more ? c + 1 : c);
-            const dn_i32x4 rq = rows_rsrc(p.q, more ? c + 1 : c);
-            const int ta = 16 * wave + l16;
-#pragma unroll
-            for (int q = 0; q < D / 32; q++) {
-                const int pos = (4 * q + g) ^ (ta & 15);
-                const uint4 ka = *(const uint4*)(kt + ta * 256 + pos * 16);
-                const uint4 qa = *(const uint4*)(qt + ta * 256 + pos * 16);
-#pragma unroll
-                for (int pc = 0; pc < 3; pc++) {
-                    const uint4 sb = Sp[(pc * (D / 32) + q) * 64 + lane];
-                    ak0 = mfma32<DT>(ka, sb, ak0);
-                    aq0 = mfma32<DT>(qa, sb, aq0);
-                }
-                if (more && q < KR) {
-                    dma_row_round(rk, kn, q);
-                    if (Q2) dma_row_round(rq, qn, q);
-                }
-            }
-            static_assert(!BF || KR <= D / 32, "the DMA rounds fit the k-steps");
-        } else {
+        {
             const dn_i32x4 rk = rows_rsrc(p.k, more ? c + 1 : c);
             const dn_i32x4 rq = rows_rsrc(p.q, more ? c + 1 : c);
             const int ta = 16 * wave + l16;
@@ -841,19 +822,6 @@ __global__ __launch_bounds__(kChunkThreads, 1) void deltanet_chunk_scan_kernel(c
 #pragma unroll
         for (int i = 0; i < 4; i++) nf |= !is_finite_f(dl[i]);
         *(float4*)(Dl + (wave * 64 + lane) * 4) = make_float4(dl[0], dl[1], dl[2], dl[3]);
-        if constexpr (BF) {
-            // the state update's B operand: Delta rows t = 16 w + 4 g + i scaled by
-            // (gamma_last / gamma_t) / |k_t|, as pieces at k-step t / 32, lane
-            // 16 ((t % 32) / 8) + n, slots t % 8
-            const float4 sk = *(const float4*)(scl + 3 * C + 16 * wave + 4 * g);
-            const float xs[4] = {dl[0] * sk.x, dl[1] * sk.y, dl[2] * sk.z, dl[3] * sk.w};
-            uint2 pcs[3];
-            dn_split3x4(xs, pcs);
-#pragma unroll
-            for (int pc = 0; pc < 3; pc++)
-                *(uint2*)((char*)&Dp[(pc * (C / 32) + (wave >> 1)) * 64 + 16 * (2 * (wave & 1) + (g >> 1)) + l16] +
-                          8 * (g & 1)) = pcs[pc];
-        }
         if (nf) flag = 1;
         dn_lds_barrier();  // Delta complete
         if (!Q2 && more) {  // the single f32 Q buffer: its reads ended with step b
@@ -894,38 +862,6 @@ __global__ __launch_bounds__(kChunkThreads, 1) void deltanet_chunk_scan_kernel(c
             dn_f32x4 a0 = gl * s0own[0], a1 = gl * s0own[1];
             dn_f32x4 b0 = {0.0f, 0.0f, 0.0f, 0.0f}, b1 = b0;
             const int j0 = 32 * wave + l16, j1 = j0 + 16;
-            if constexpr (BF) {
-                // A = K^T (state rows 32 w + 16 tt + 0..15, tokens 32 ks + 8 g .. + 7):
-                // two transposing reads of 4 tokens x 16 dims each (lane i of a
-                // 16-lane group supplies token k0 + i / 4, dims d0 + 4 (i % 4) .. + 3,
-                // and receives dims d0 + i of tokens k0 .. k0 + 3); B = the pieces of
-                // the scaled Delta
-#pragma unroll
-                for (int ks = 0; ks < C / 32; ks++) {
-                    uint4 at[2];
-#pragma unroll
-                    for (int tt = 0; tt < 2; tt++) {
-                        dn_s4 part[2];
-#pragma unroll
-                        for (int hf = 0; hf < 2; hf++) {
-                            const int t = 32 * ks + 8 * g + 4 * hf + (l16 >> 2);
-                            const int e = 32 * wave + 16 * tt + 4 * (l16 & 3);
-                            const int pos = (e >> 3) ^ (t & 15);
-                            part[hf] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                                (__attribute__((address_space(3))) dn_s4*)(kt + t * 256 + pos * 16 + (e & 7) * 2));
-                        }
-                        const uint2 lo2 = __builtin_bit_cast(uint2, part[0]);
-                        const uint2 hi2 = __builtin_bit_cast(uint2, part[1]);
-                        at[tt] = make_uint4(lo2.x, lo2.y, hi2.x, hi2.y);
-                    }
-#pragma unroll
-                    for (int pc = 0; pc < 3; pc++) {
-                        const uint4 db = Dp[(pc * (C / 32) + ks) * 64 + lane];
-                        a0 = mfma32<DT>(at[0], db, a0);
-                        a1 = mfma32<DT>(at[1], db, a1);
-                    }
-                }
-            } else {
 #pragma unroll
             for (int q = 0; q < C / 16; q++) {
                 const float4 b = *(const float4*)(Dl + (q * 64 + lane) * 4);
@@ -941,17 +877,12 @@ __global__ __launch_bounds__(kChunkThreads, 1) void deltanet_chunk_scan_kernel(c
                 b0 = mfma4(dn_elem<DT>(kt, s + 3, j0), bs[3], b0);
                 b1 = mfma4(dn_elem<DT>(kt, s + 3, j1), bs[3], b1);
             }
-            }
             a0 += b0;
             a1 += b1;
 #pragma unroll
             for (int i = 0; i < 4; i++) nf |= !is_finite_f(a0[i]) || !is_finite_f(a1[i]);
             *(float4*)srow0 = make_float4(a0[0], a0[1], a0[2], a0[3]);
             *(float4*)srow1 = make_float4(a1[0], a1[1], a1[2], a1[3]);
-            if constexpr (BF) {
-                const float v0[4] = {a0[0], a0[1], a0[2], a0[3]}, v1[4] = {a1[0], a1[1], a1[2], a1[3]};
-                store_state_pieces(v0, v1);
-            }
         }
         if (nf) flag = 1;
 #pragma unroll
@@ -985,10 +916,414 @@ __global__ __launch_bounds__(kChunkThreads, 1) void deltanet_chunk_scan_kernel(c
     if (tid == 0) ((int*)p.ws)[h * kScanBlocks + cb] = done;
 }
 
+// bf16 rows.  One workgroup of eight waves per (head, 16 state columns), the chunks in
+// order, as above, but chain wave w < 4 keeps state rows 32 w .. 32 w + 31 in registers,
+// both as f32 MFMA results and, cut into three exact bf16 pieces, as the B operand of
+// k-step w: its two result tiles take rows 32 w + 8 g + 4 tt + i, so a lane's results
+// are its own operand slots and the state does not pass through LDS on its way to
+// the next chunk.  Products over the 128 state rows are then sums over the waves.  Per
+// chunk the chain waves compute
+//   1. K S0 over the wave's 32 rows, all 64 tokens                -> LDS (partial sums)
+//   2. X = beta V - (beta gamma / |k|) sum_w (K S0)_w, 16 tokens   -> LDS (pieces)
+//   3. Delta = T X, 16 tokens, plain                               -> LDS (f32)
+//      and scaled by (gamma_last / gamma) / |k|                    -> LDS (pieces)
+//   4. S' = gamma_last S0 + K^T (scaled Delta), 32 rows            -> LDS (pieces)
+// with a barrier after each of 1 - 3, and the output waves 4 .. 7 follow beside them,
+// 16 tokens each: Q S0 beside step 3, O = (gamma / |q| sqrt(d)) Q S0 + P Delta beside
+// step 4.  f32 x f32 products take the six piece products down to 2^-16 (hi
+// hi, hi mid, mid hi, hi lo, mid mid, lo hi), bf16 x f32 ones all three (a bf16 MFMA
+// has 8 times the reduction length of an f32 one at half its time); P Delta stays on
+// the f32 MFMA.  Global operands go straight into registers, each loaded for the next
+// chunk right after its last use in this one; K^T comes from the wave's own K
+// fragments through LDS.  What bounds it: the dependent steps of one chunk (LDS
+// round trips, barriers, the VALU work of cutting values into pieces) and the output
+// waves' products on the same SIMDs.  MI355X, 4096 tokens, 16 heads: 174 -> 122 us
+// (the chain waves alone 100; Q S0 and P Delta by the chain waves themselves, with
+// every operand loaded from memory, 210; P Delta beside step 2 147).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t bf_rsrc(const char* base, int bytes) {
+    // (uniform values that the compiler may hold in vector registers)
+    const uint64_t a = (uint64_t)(uintptr_t)base;
+    const uint64_t u = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a) |
+                       (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) << 32;
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)u, 0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+}
+__device__ __forceinline__ uint4 bf_load16(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+}
+__device__ __forceinline__ float4 bf_load4f(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+    return __builtin_bit_cast(float4, bf_load16(r, voff, soff));
+}
+__device__ __forceinline__ dn_f32x4 bf_mma(const uint4& a, const uint4& b, dn_f32x4 c) {
+    return mfma32<GR_DTYPE_BF16>(a, b, c);
+}
+// six piece products of A (a[0..2]) and B (b[0..2]): three chains
+__device__ __forceinline__ void bf_mma6(const uint4* a, const uint4* b, dn_f32x4* acc) {
+    acc[0] = bf_mma(a[0], b[0], acc[0]);
+    acc[1] = bf_mma(a[0], b[1], acc[1]);
+    acc[2] = bf_mma(a[1], b[0], acc[2]);
+    acc[1] = bf_mma(a[0], b[2], acc[1]);
+    acc[2] = bf_mma(a[1], b[1], acc[2]);
+    acc[1] = bf_mma(a[2], b[0], acc[1]);
+}
+
+constexpr int kBfThreads = 512;
+
+__global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel(const DeltaNetLaunch p) {
+    constexpr int C = kChunk, D = 128, NC = kScanCols;
+    __shared__ __attribute__((aligned(16))) float4 Pk[4][4][64];  // [token tile][wave][lane]
+    __shared__ __attribute__((aligned(16))) uint4 Xp[2][3][64];   // [k-step][piece][lane]
+    __shared__ __attribute__((aligned(16))) uint4 Ds[2][3][64];   // scaled Delta
+    __shared__ __attribute__((aligned(16))) float4 Dl[4][64];     // Delta [wave][lane]
+    __shared__ __attribute__((aligned(16))) uint4 Sp[4][3][64];   // state [k-step][piece][lane]
+    // K of a chain wave's 32 dims: token t's 16-byte chunk c at c ^ (t / 8 % 4)
+    __shared__ __attribute__((aligned(16))) char Kl[4][C * 64];
+    __shared__ int flag;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = wave8 & 3;
+    const int l16 = lane & 15, g = lane >> 4;
+    const int h = blockIdx.x, cb = blockIdx.y;  // as above: one head's column blocks share an XCD
+    const int c0 = cb * NC;
+    const int H = p.n_heads;
+    float* Sh = p.state + (size_t)h * D * D;
+    const int n_chunks = (p.n_tokens + C - 1) / C;
+    const int row = H * D * 2;  // bytes between token rows of q / k / v
+    const dn_f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+
+    // The loads run one chunk ahead: `roff` is the byte offset of the next chunk's rows
+    // in q / k / v, `rbytes` the bytes of its rows (rows past the end of the sequence,
+    // and every row past the last chunk, read as zero: they are past the descriptor),
+    // `blk` / `bbytes` its block.
+    size_t roff = (size_t)h * D * 2;
+    int left = p.n_tokens, rbytes = 0, bbytes = kBfBytes;
+    const char* blk = (const char*)p.ws + dn_ws_head(H) + (size_t)h * kBfBytes;
+    auto bytes_of = [&]() { return left > 0 ? (min(C, left) - 1) * row + D * 2 : 0; };
+    rbytes = bytes_of();
+    auto next_chunk = [&]() {
+        roff += (size_t)C * row;
+        blk += (size_t)H * kBfBytes;
+        left -= C;
+        rbytes = bytes_of();
+        bbytes = left > 0 ? kBfBytes : 0;
+    };
+    auto rows_of = [&](const void* src) { return bf_rsrc((const char*)src + roff, rbytes); };
+    auto block_of = [&]() { return bf_rsrc(blk, bbytes); };
+    // gamma_last, flag
+    auto load_gl = [&]() { return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(block_of(), 0, kBfGl, 0)); };
+
+    if (tid == 0) flag = 0;
+    int done = n_chunks;  // chunks completed
+    int c = 0;
+    bool all = true, back = false;
+    // Both roles leave the loop at the same place: after the third barrier of a chunk that
+    // the prep flagged (its state rows are not updated yet), or after the first barrier of
+    // a chunk whose predecessor met a non-finite value (which is then resumed from its
+    // own start).  They wait for their loads on the way out: the compiler's waits in the
+    // loop, which shares its last block with the exits, then need not cover them.
+    auto flagged = [&](uint2 gb) { return __builtin_amdgcn_readfirstlane((int)gb.y) != 0; };
+    auto failed = [&]() { return __builtin_amdgcn_readfirstlane(flag) != 0; };
+#define DN_BF_LEAVE(at, to_start) { dn_wait_vmem(); all = false; done = (at); back = (to_start); break; }
+
+    if (wave8 >= 4) {
+        // output waves: tokens 16 w + m
+        int qoff[4], dlane[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            qoff[q] = (16 * wave + l16) * row + (32 * q + 8 * g) * 2;
+            // Delta of tokens 16 q + 4 g + i: chain wave 2 (q / 2) + g % 2
+            dlane[q] = (2 * (q >> 1) + (g & 1)) * 64 + 16 * (2 * (q & 1) + (g >> 1)) + l16;
+        }
+        const int orow = H * D * 4;
+        const int ooff = (16 * wave + 4 * g) * orow + (c0 + l16) * 4;
+        uint4 qa[4];
+        float4 pa[4], sq;
+        uint2 gb;
+        const int apos = 16 * (4 * l16 + (g ^ ((l16 >> 2) & 3)));  // this lane's piece in a P tile
+        auto load_q = [&]() {
+            const auto r = rows_of(p.q);
+#pragma unroll
+            for (int q = 0; q < 4; q++) qa[q] = bf_load16(r, qoff[q], 0);
+        };
+        auto load_p = [&]() {
+            const auto r = block_of();
+#pragma unroll
+            for (int q = 0; q < 4; q++)  // past the diagonal: past the block, zero
+                pa[q] = bf_load4f(r, apos, q <= wave ? kBfP + tp_tri(wave, q) * 1024 : kBfBytes);
+            sq = bf_load4f(r, 4 * (16 * wave + 4 * g), kBfScale + 8 * C);
+        };
+        // O of chunk n and its store, from Q S0 (aq) and the chunk's Delta
+        dn_f32x4 aq[2];
+        const char* ob = (const char*)p.out + (size_t)h * D * 4;  // rows of the chunk to finish
+        int oleft = p.n_tokens;
+        auto finish = [&]() {
+            dn_f32x4 o0 = zero, o1 = zero;
+            float4 b[4];
+#pragma unroll
+            for (int q = 0; q < 4; q++) b[q] = ((const float4*)Dl)[dlane[q]];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                o0 = mfma4(pa[q].x, b[q].x, o0);
+                o1 = mfma4(pa[q].y, b[q].y, o1);
+                o0 = mfma4(pa[q].z, b[q].z, o0);
+                o1 = mfma4(pa[q].w, b[q].w, o1);
+            }
+            const float s4[4] = {sq.x, sq.y, sq.z, sq.w};
+            // (rows past the end are past the descriptor: not stored)
+            const auto r = bf_rsrc(ob, (min(C, oleft) - 1) * orow + D * 4);
+            float nf = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float ov = s4[i] * (aq[0][i] + aq[1][i]) + (o0[i] + o1[i]);
+                nf = fmaf(ov, 0.0f, nf);  // x * 0 is NaN for an infinity or a NaN
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ov), r, ooff + i * orow, 0, 0);
+            }
+            if (nf != 0.0f) flag = 1;
+            ob += (size_t)C * orow;
+            oleft -= C;
+        };
+        gb = load_gl();
+        __builtin_amdgcn_sched_barrier(0);
+        load_q();
+        __builtin_amdgcn_sched_barrier(0);
+        load_p();
+        __builtin_amdgcn_sched_barrier(0);
+        next_chunk();
+        dn_lds_barrier();
+        for (; c < n_chunks; c++) {
+            dn_lds_barrier();  // 1
+            if (failed()) DN_BF_LEAVE(c - 1, true);
+            dn_lds_barrier();  // 2
+            {
+                uint4 sb[4][3];
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+#pragma unroll
+                    for (int pc = 0; pc < 3; pc++) sb[q][pc] = Sp[q][pc][lane];
+                aq[0] = aq[1] = zero;
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+#pragma unroll
+                    for (int pc = 0; pc < 3; pc++) aq[q & 1] = bf_mma(qa[q], sb[q][pc], aq[q & 1]);
+            }
+            load_q();
+            dn_lds_barrier();  // 3
+            if (flagged(gb)) DN_BF_LEAVE(c, false);
+            gb = load_gl();
+            finish();
+            load_p();
+            next_chunk();
+        }
+        if (all) dn_lds_barrier();
+        return;
+    }
+
+    // chain waves
+    __builtin_amdgcn_s_setprio(2);  // they bound the chunk
+    const int tok0 = bf_tok(wave, 4 * g);  // the lane's tokens: tok0 .. tok0 + 3
+    int koff[4], voff[4];
+#pragma unroll
+    for (int mt = 0; mt < 4; mt++) koff[mt] = bf_tok(mt, l16) * row + (32 * wave + 8 * g) * 2;
+#pragma unroll
+    for (int i = 0; i < 4; i++) voff[i] = (tok0 + i) * row + (c0 + l16) * 2;
+    // T operands of k-steps 0 and 1 (w < 2 has no k-step 1: past the block, zero)
+    const int toff[2] = {kBfT + 3072 * (wave < 2 ? wave : 2 * wave - 2), wave < 2 ? kBfBytes : kBfT + 3072 * (2 * wave - 1)};
+    char* kl = Kl[wave];
+    uint4 ka[4], ta[2][3];
+    float4 sb, sx, sk;
+    uint32_t vr[4];
+    uint2 gb;
+    auto load_k = [&]() {
+        const auto r = rows_of(p.k);
+#pragma unroll
+        for (int mt = 0; mt < 4; mt++) ka[mt] = bf_load16(r, koff[mt], 0);
+    };
+    auto load_x = [&]() {
+        const auto r = block_of();
+        sb = bf_load4f(r, 4 * tok0, kBfScale);
+        sx = bf_load4f(r, 4 * tok0, kBfScale + 4 * C);
+        const auto v = rows_of(p.v);
+#pragma unroll
+        for (int i = 0; i < 4; i++) vr[i] = __builtin_amdgcn_raw_buffer_load_b16(v, voff[i], 0, 0);
+    };
+    auto load_t = [&]() {
+        const auto r = block_of();
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+            for (int pc = 0; pc < 3; pc++) ta[ks][pc] = bf_load16(r, 16 * lane, toff[ks] + 1024 * pc);
+        sk = bf_load4f(r, 4 * tok0, kBfScale + 12 * C);
+    };
+    // four values of the lane as slots 4 (w % 2) .. + 3 of lane (g, l % 16) of k-step w / 2
+    auto put = [&](uint4 (*dst)[3][64], const float* x) {
+        uint2 pcs[3];
+        dn_split3x4(x, pcs);
+#pragma unroll
+        for (int pc = 0; pc < 3; pc++) *((uint2*)&dst[wave >> 1][pc][lane] + (wave & 1)) = pcs[pc];
+    };
+    // the wave's state rows 32 w + 8 g + 4 tt + i of column c0 + l16
+    dn_f32x4 st[2], s0own[2];
+    uint4 sp[3];
+    auto split_state = [&]() {
+        uint2 a[3], b[3];
+        const float x0[4] = {st[0][0], st[0][1], st[0][2], st[0][3]}, x1[4] = {st[1][0], st[1][1], st[1][2], st[1][3]};
+        dn_split3x4(x0, a);
+        dn_split3x4(x1, b);
+#pragma unroll
+        for (int pc = 0; pc < 3; pc++) {
+            sp[pc] = make_uint4(a[pc].x, a[pc].y, b[pc].x, b[pc].y);
+            Sp[wave][pc][lane] = sp[pc];
+        }
+    };
+#pragma unroll
+    for (int tt = 0; tt < 2; tt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) st[tt][i] = Sh[(size_t)(32 * wave + 8 * g + 4 * tt + i) * D + c0 + l16];
+    s0own[0] = st[0], s0own[1] = st[1];
+    split_state();
+    // the first chunk's loads in the loop's order (its waits count the loads behind an
+    // operand on both ways into the loop)
+    gb = load_gl();
+    __builtin_amdgcn_sched_barrier(0);
+    load_k();
+    __builtin_amdgcn_sched_barrier(0);
+    load_x();
+    __builtin_amdgcn_sched_barrier(0);
+    load_t();
+    __builtin_amdgcn_sched_barrier(0);
+    next_chunk();
+    dn_lds_barrier();
+    for (; c < n_chunks; c++) {
+        // 1.
+        dn_f32x4 ak[4];
+#pragma unroll
+        for (int pc = 0; pc < 3; pc++)
+#pragma unroll
+            for (int mt = 0; mt < 4; mt++) ak[mt] = bf_mma(ka[mt], sp[pc], pc ? ak[mt] : zero);
+#pragma unroll
+        for (int mt = 0; mt < 4; mt++) {
+            const int t = bf_tok(mt, l16);
+            *(uint4*)(kl + t * 64 + 16 * (g ^ ((t >> 3) & 3))) = ka[mt];
+        }
+        load_k();
+#pragma unroll
+        for (int mt = 0; mt < 4; mt++) Pk[mt][wave][lane] = make_float4(ak[mt][0], ak[mt][1], ak[mt][2], ak[mt][3]);
+        dn_lds_barrier();  // 1
+        // 2.
+        {
+            float4 pk[4];
+#pragma unroll
+            for (int w = 0; w < 4; w++) pk[w] = Pk[wave][w][lane];
+            // (the sums' reads stay above the flag's branch)
+#pragma unroll
+            for (int w = 0; w < 4; w++) asm volatile("" : "+v"(pk[w].x), "+v"(pk[w].y), "+v"(pk[w].z), "+v"(pk[w].w));
+            if (failed()) DN_BF_LEAVE(c - 1, true);
+            const float ks[4] = {(pk[0].x + pk[1].x) + (pk[2].x + pk[3].x), (pk[0].y + pk[1].y) + (pk[2].y + pk[3].y),
+                                 (pk[0].z + pk[1].z) + (pk[2].z + pk[3].z), (pk[0].w + pk[1].w) + (pk[2].w + pk[3].w)};
+            const float b4[4] = {sb.x, sb.y, sb.z, sb.w}, x4[4] = {sx.x, sx.y, sx.z, sx.w};
+            float xv[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                // (the conversion stays here: it would wait for the load in the chunk before)
+                asm volatile("" : "+v"(vr[i]));
+                xv[i] = b4[i] * __uint_as_float(vr[i] << 16) - x4[i] * ks[i];
+            }
+            put(Xp, xv);
+        }
+        load_x();
+        dn_lds_barrier();  // 2
+        // 3.
+        uint4 kt[2][2];
+        {
+            dn_f32x4 acc[3] = {zero, zero, zero};
+            uint4 xb[2][3];
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+                for (int pc = 0; pc < 3; pc++) xb[ks][pc] = Xp[ks][pc][lane];
+            __builtin_amdgcn_sched_barrier(0);  // every read issued before the first product
+            bf_mma6(ta[0], xb[0], acc);
+            bf_mma6(ta[1], xb[1], acc);
+            // K^T (rows 8 m / 4 + 4 tt + m % 4 of the wave's dims, tokens 32 ks + 8 g ..): lane i
+            // of a 16-lane group supplies token k0 + i / 4, half tt of chunk i % 4, and
+            // receives dim i of the four chunks' halves
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+                for (int tt = 0; tt < 2; tt++) {
+                    uint2 part[2];
+#pragma unroll
+                    for (int hf = 0; hf < 2; hf++) {
+                        const int t = 32 * ks + 8 * g + 4 * hf + (l16 >> 2);
+                        part[hf] = __builtin_bit_cast(
+                            uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) dn_s4*)(
+                                       kl + t * 64 + 16 * ((l16 & 3) ^ g) + 8 * tt)));
+                    }
+                    kt[tt][ks] = make_uint4(part[0].x, part[0].y, part[1].x, part[1].y);
+                }
+            const dn_f32x4 dl = acc[0] + (acc[1] + acc[2]);
+            const float k4[4] = {sk.x, sk.y, sk.z, sk.w};
+            float ds[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                ds[i] = dl[i] * k4[i];
+            }
+            put(Ds, ds);
+            Dl[wave][lane] = make_float4(dl[0], dl[1], dl[2], dl[3]);
+        }
+        load_t();
+        dn_lds_barrier();  // 3
+        // 4.
+        {
+            if (flagged(gb)) DN_BF_LEAVE(c, false);
+            const float gl = __uint_as_float(gb.x);
+            float nf = 0.0f;
+            uint4 db[2][3];
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+                for (int pc = 0; pc < 3; pc++) db[ks][pc] = Ds[ks][pc][lane];
+            __builtin_amdgcn_sched_barrier(0);
+            s0own[0] = st[0], s0own[1] = st[1];
+            dn_f32x4 a0 = gl * st[0], a1 = gl * st[1], b0 = zero, b1 = zero;
+            gb = load_gl();
+#pragma unroll
+            for (int pc = 0; pc < 3; pc++) {
+                a0 = bf_mma(kt[0][0], db[0][pc], a0);
+                a1 = bf_mma(kt[1][0], db[0][pc], a1);
+                b0 = bf_mma(kt[0][1], db[1][pc], b0);
+                b1 = bf_mma(kt[1][1], db[1][pc], b1);
+            }
+            st[0] = a0 + b0;
+            st[1] = a1 + b1;
+#pragma unroll
+            for (int i = 0; i < 4; i++) nf = fmaf(st[1][i], 0.0f, fmaf(st[0][i], 0.0f, nf));
+            split_state();
+            if (nf != 0.0f) flag = 1;
+        }
+        // x * 0 is NaN for an infinity or a NaN.  A non-finite X gives a non-finite Delta
+        // (T has a unit diagonal), and that non-finite state rows.
+        next_chunk();
+    }
+    if (all) {
+        dn_lds_barrier();
+        if (flag) {  // the last chunk met a non-finite value
+            done = n_chunks - 1;
+            back = true;
+        }
+    }
+#undef DN_BF_LEAVE
+#pragma unroll
+    for (int tt = 0; tt < 2; tt++)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            Sh[(size_t)(32 * wave + 8 * g + 4 * tt + i) * D + c0 + l16] = back ? s0own[tt][i] : st[tt][i];
+    if (tid == 0) ((int*)p.ws)[h * kScanBlocks + cb] = done;
+}
+
 size_t deltanet_chunked_ws_bytes(int n_tokens, int n_heads, int head_dim, int chunk) {
     if (head_dim != 128 || chunk != kChunk || n_tokens <= 0 || n_heads <= 0) return 0;
     const size_t n_chunks = (size_t)(n_tokens + kChunk - 1) / kChunk;
-    return dn_ws_head(n_heads) + n_chunks * n_heads * kTpBytes;
+    return dn_ws_head(n_heads) + n_chunks * n_heads * kBfBytes;  // (the larger of the two blocks)
 }
 
 // The token recurrence at any supported state size (64, 128, 256: 32 value
@@ -1017,7 +1352,9 @@ static hipError_t launch_chunked_dt(const DeltaNetLaunch& p, hipStream_t st) {
     deltanet_chunk_prep_kernel<DT><<<dim3(n_chunks, p.n_heads), kChunkThreads, lds_prep, st>>>(p);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
-    deltanet_chunk_scan_kernel<DT><<<dim3(p.n_heads, kScanBlocks), kChunkThreads, 0, st>>>(p);
+    const dim3 grid(p.n_heads, kScanBlocks);
+    if constexpr (DT == GR_DTYPE_BF16) deltanet_chunk_scan_bf16_kernel<<<grid, kBfThreads, 0, st>>>(p);
+    else deltanet_chunk_scan_kernel<DT><<<grid, kChunkThreads, 0, st>>>(p);
     return hipGetLastError();
 }
 

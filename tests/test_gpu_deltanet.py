@@ -153,6 +153,53 @@ def test_deltanet_16bit_inputs_chunked(orc, dev, fmt, l2norm):
     assert float(np.abs(S - Sref).max()) <= TOL, np.abs(S - Sref).max()
 
 
+@pytest.mark.parametrize("T", [1, 63, 64, 65, 128, 129, 321])
+def test_deltanet_bf16_scan_chunk_edges(orc, dev, T):
+    """The bf16 scan (state in registers, operands loaded a chunk ahead): one chunk, whole
+    chunks, one row past a chunk, odd and even chunk counts; f32 arithmetic bar."""
+    rng = np.random.default_rng(T)
+    S0 = (0.1 * rng.standard_normal((3, 128, 128))).astype(np.float32)
+    got, ref, S, Sref = _run(orc, dev, T, 3, 128, 40 + T, orc.BF16, 2, state0=S0)
+    assert float(np.abs(got - ref).max()) <= TOL, np.abs(got - ref).max()
+    assert float(np.abs(S - Sref).max()) <= TOL, np.abs(S - Sref).max()
+
+
+def test_deltanet_bf16_scan_nonfinite(orc, dev):
+    """Non-finite values in the bf16 scan: inputs (flagged by the prep, in the first, a
+    middle and the ragged last chunk) and a state column that overflows inside the scan
+    (gates above zero): its column block continues token by token from that chunk.
+    Every other column keeps the f32 bar; the overflowing one only stays finite (where
+    a sum overflows depends on its order)."""
+    T, H, d = 500, 6, 128
+    q, k, v, gate, beta = _inputs(orc, T, H, d, 99, orc.BF16)
+    nan, inf = orc.bf16_bits(np.array([np.nan, np.inf], np.float32))
+    v[3, 0, 7] = nan
+    k[200, 1, 11] = inf
+    q[499, 2, 0] = nan
+    gate[260, 3] = np.nan
+    S0 = (0.05 * np.random.default_rng(1).standard_normal((H, d, d))).astype(np.float32)
+    gate[:300, 4] = 0.15
+    gate[300, 4] = -90.0
+    S0[4, :, 21] = 1e33
+    ref, Sref = orc.deltanet_scan(*(orc.upcast(x, orc.BF16) for x in (q, k, v)), gate, beta, S0, eps=1e-6,
+                                  n_threads=orc.env_threads())
+    from gguf_runner_amd import ops
+    st = torch.from_numpy(S0.copy()).to(dev)
+    out = torch.empty((T, H, d), dtype=torch.float32, device=dev)
+    ops.DeltaNetCall(*(_to_dev(x, orc.BF16, orc, dev) for x in (q, k, v)), torch.from_numpy(gate).to(dev),
+                     torch.from_numpy(beta).to(dev), st, out, algo=2)()
+    torch.cuda.synchronize()
+    got, S = out.cpu().numpy(), st.cpu().numpy()
+    assert np.isfinite(got).all()
+    cols = np.ones((H, d), bool)
+    cols[4, 21] = False
+    # head 4's other columns grow with the gates too (to ~1e17): relative to their size
+    tol = TOL * np.maximum(1.0, np.abs(np.where(cols, ref, 0)).max(axis=2, keepdims=True))
+    assert (np.abs(got - ref) <= tol)[:, cols].all()
+    bad = np.abs(S - Sref) > TOL * np.maximum(1.0, np.abs(Sref))
+    assert not bad.transpose(0, 2, 1)[cols].any()
+
+
 @pytest.mark.parametrize("d,algo,fmt_name", [(64, 1, "F32"), (64, 0, "BF16"), (256, 1, "F32"), (256, 2, "F16")])
 def test_deltanet_state_sizes_64_and_256(orc, dev, d, algo, fmt_name):
     """State sizes other than 128 (the reference takes any ssm_state_size, math.rs:566):
