@@ -20,7 +20,8 @@
 //    which is the token recurrence whenever every guard of the reference is a
 //    no-op (all values finite).
 //    deltanet_chunk_prep_kernel (chunk, head): T, P and per-row scales; the
-//    Gram products on v_mfma_f32_16x16x4_f32, T by forward substitution.
+//    Gram products on v_mfma_f32_16x16x4_f32, T by forward substitution in the
+//    diagonal 16x16 blocks and products below them.
 //    deltanet_chunk_scan_kernel (head, 16 state columns): the sequential chunk
 //    steps with the raw q / k rows as operands and their row scales applied to
 //    the products' rows; T X and P Delta on v_mfma_f32_16x16x4_f32, and K S0,
@@ -289,7 +290,8 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
     uint16_t* qr = (uint16_t*)smem;            // 16-bit: [C][RS16] raw q rows
     uint16_t* kr = qr + C * RS16;              // 16-bit: [C][RS16] raw k rows
     float* am = smem;                          // [C][AMS] A (strictly lower), over the rows once the products are done
-    static_assert(C * AMS * 4 <= dn_prep_lds<DT>(), "A fits over the rows");
+    float* tm = am + C * AMS;                  // [C][AMS] T (its diagonal blocks; bf16: all of it)
+    static_assert(2 * C * AMS * 4 <= dn_prep_lds<DT>(), "A and T fit over the rows");
     // in-chunk cumulative log decay in double: with strong decays the prefix sums
     // reach ~-100 within a chunk, and a decay exp(lg[t] - lg[s]) taken from two
     // f32 prefix sums would carry ~100 ulp of absolute error in its exponent
@@ -447,46 +449,66 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
     }
     __syncthreads();
 
-    // 3. T = (I + A)^-1, column col = 16 wave + lane / 4 by forward substitution
-    //    x[t] = [t == col] - sum_{s<t} A[t][s] x[s]; the four lanes of a quad
-    //    take the 4-blocks of s with (s / 4) % 4 == part and sum by DPP.
+    // 3. T = (I + A)^-1 in 16x16 blocks.  Wave w inverts the diagonal block w by forward
+    //    substitution (16 steps; 64 steps over whole columns took two thirds of this
+    //    kernel's VALU instructions), then takes block column w down on the f32 MFMA:
+    //    T[i][w] = -T[i][i] sum_{w <= k < i} A[i][k] T[k][w].  A result (row 4 g + e,
+    //    column l % 16) is the next product's B operand as it stands.
     {
-        const int col = 16 * wave + (lane >> 2), part = lane & 3;
-        float x[16];  // x[s] for s = 16 u + 4 part + e at x[4 u + e]
+        // column col of the block: x[t] = [t == col] - sum_{s<t} A[t][s] x[s]; the four
+        // lanes of a quad take s = 4 part .. + 3 and sum by DPP
+        const int col = lane >> 2, part = lane & 3;
+        const float* ad = am + 16 * wave * AMS + 16 * wave + 4 * part;
+        float x[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int e = 0; e < 16; e++) x[e] = 0.0f;
-#pragma unroll
-        for (int t = 0; t < C; t++) {
-            float su[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // four short chains instead of one long one
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                if (16 * u < t) {  // A[t][s >= t] is 0 and x[s >= t] is still 0
-                    const float4 a = *(const float4*)(am + t * AMS + 16 * u + 4 * part);
-                    su[u] = a.x * x[4 * u + 0];
-                    su[u] = fmaf(a.y, x[4 * u + 1], su[u]);
-                    su[u] = fmaf(a.z, x[4 * u + 2], su[u]);
-                    su[u] = fmaf(a.w, x[4 * u + 3], su[u]);
-                }
-            }
-            const float sum = quad_sum((su[0] + su[1]) + (su[2] + su[3]));
+        for (int t = 0; t < 16; t++) {
+            const float4 a = *(const float4*)(ad + t * AMS);  // A[t][s >= t] is 0
+            const float sum = quad_sum(fmaf(a.x, x[0], a.y * x[1]) + fmaf(a.z, x[2], a.w * x[3]));
             const float val = (t == col ? 1.0f : 0.0f) - sum;
-            // a select, not a branch: under a lane-dependent branch the compiler
-            // copied the whole x array at every step
-            const int xi = (t >> 4) * 4 + (t & 3);
-            x[xi] = ((t >> 2) & 3) == part ? val : x[xi];
+            // a select, not a branch
+            x[t & 3] = (t >> 2) == part ? val : x[t & 3];
         }
-        if constexpr (BF) __syncthreads();  // every read of A is done: T goes over it
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            if (!BF && u < wave) continue;  // T[s][col] = 0 above the diagonal tiles
+        for (int e = 0; e < 4; e++) {
+            if (!is_finite_f(x[e])) bad = 1;
+            tm[(16 * wave + 4 * part + e) * AMS + 16 * wave + col] = x[e];
+            if constexpr (!BF) *(float*)(blk + kTpT + tp_tri(wave, wave) * 1024 + 4 * tp_elem(4 * part + e, col)) = x[e];
+        }
+        __syncthreads();
+        dn_f32x4 tb[4];  // T[i][wave]
+#pragma unroll
+        for (int e = 0; e < 4; e++) tb[0][e] = tm[(16 * wave + 4 * g + e) * AMS + 16 * wave + l16];
+#pragma unroll
+        for (int n = 1; n < 4; n++) {  // block row i = wave + n
+            const int i = wave + n;
+            if (i > 3) break;
+            dn_f32x4 y0 = {0.0f, 0.0f, 0.0f, 0.0f}, y1 = y0;
+#pragma unroll
+            for (int k = 0; k < n; k++) {
+                const float4 a = *(const float4*)(am + (16 * i + l16) * AMS + 16 * (wave + k) + 4 * g);
+                y0 = mfma4(a.x, tb[k][0], y0);
+                y1 = mfma4(a.y, tb[k][1], y1);
+                y0 = mfma4(a.z, tb[k][2], y0);
+                y1 = mfma4(a.w, tb[k][3], y1);
+            }
+            y0 += y1;
+            const float4 d = *(const float4*)(tm + (16 * i + l16) * AMS + 16 * i + 4 * g);
+            dn_f32x4 z0 = {0.0f, 0.0f, 0.0f, 0.0f}, z1 = z0;
+            z0 = mfma4(d.x, y0[0], z0);
+            z1 = mfma4(d.y, y0[1], z1);
+            z0 = mfma4(d.z, y0[2], z0);
+            z1 = mfma4(d.w, y0[3], z1);
+            tb[n] = -(z0 + z1);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                const float v = x[4 * u + e];
-                if (!is_finite_f(v)) bad = 1;
-                if constexpr (BF) am[(16 * u + 4 * part + e) * AMS + col] = v;
-                else *(float*)(blk + kTpT + tp_tri(u, wave) * 1024 + 4 * tp_elem(4 * part + e, lane >> 2)) = v;
+                if (!is_finite_f(tb[n][e])) bad = 1;
+                if constexpr (BF) tm[(16 * i + 4 * g + e) * AMS + 16 * wave + l16] = tb[n][e];
+                else *(float*)(blk + kTpT + tp_tri(i, wave) * 1024 + 4 * tp_elem(4 * g + e, l16)) = tb[n][e];
             }
         }
+        // the two blocks above the diagonal that T's operands read
+        if (BF && wave == 3)
+            for (int e = lane; e < 512; e += 64) tm[((e >> 8) * 32 + ((e >> 4) & 15)) * AMS + (e >> 8) * 32 + 16 + (e & 15)] = 0.0f;
     }
     if constexpr (BF) {
         __syncthreads();
@@ -496,7 +518,7 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
             const int op = wave + 4 * u;
             if (op >= 6) break;
             const int w = op < 2 ? op : (op + 2) >> 1, ks = op < 2 ? 0 : op & 1;
-            const float* src = am + bf_tok(w, l16) * AMS + 32 * ks + 8 * g;
+            const float* src = tm + bf_tok(w, l16) * AMS + 32 * ks + 8 * g;
             uint2 lo[3], hi[3];
             dn_split3x4(src, lo);
             dn_split3x4(src + 4, hi);
