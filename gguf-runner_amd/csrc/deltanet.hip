@@ -207,6 +207,15 @@ __device__ __forceinline__ float quad_sum(float v) {
     return v;
 }
 
+// Sum over the 16 lanes of a row (DPP row_ror 8, 4, 2, 1).
+__device__ __forceinline__ float row16_sum(float v) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, false));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xF, 0xF, false));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xF, 0xF, false));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xF, 0xF, false));
+    return v;
+}
+
 // MFMA 16x16x4 f32 operands: lane l holds A[l % 16][l / 16] and B[l / 16][l % 16];
 // the result holds D[4 (l / 16) + i][l % 16] in element i.  Every product below
 // gives lane group g = l / 16 the reduction indices 16 q + 4 g + i (i = 0..3)
@@ -319,10 +328,10 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
                                              8 * l16)
                            : make_uint4(0, 0, 0, 0);
         }
+        float mine = 0.0f;  // lane r4 of a row's 16 lanes keeps the sum of round r4
 #pragma unroll
         for (int r4 = 0; r4 < 8; r4++) {
             const int t = 16 * wave + 4 * (r4 & 3) + g;
-            const bool isq = r4 < 4, valid = t < Cn;
             const uint32_t w[4] = {x[r4].x, x[r4].y, x[r4].z, x[r4].w};
             float ss = 0.0f;
 #pragma unroll
@@ -331,14 +340,16 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
                 ss = fmaf(lo, lo, ss);
                 ss = fmaf(hi, hi, ss);
             }
-#pragma unroll
-            for (int m = 1; m < 16; m <<= 1) ss += shfl_xor(ss, m);
-            *(uint4*)((isq ? qr : kr) + t * RS16 + 8 * l16) = x[r4];
-            if (l16 == 0) {
-                const float inv = 1.0f / sqrtf(ss + p.eps);
-                (isq ? qi : ki)[t] = !valid ? 0.0f : !p.l2norm ? 1.0f : isq ? inv * inv_scale_q : inv;
-                if (valid && !is_finite_f(ss)) bad = 1;
-            }
+            ss = row16_sum(ss);
+            mine = l16 == r4 ? ss : mine;
+            *(uint4*)((r4 < 4 ? qr : kr) + t * RS16 + 8 * l16) = x[r4];
+        }
+        if (l16 < 8) {  // the eight rounds' norms in eight lanes at once
+            const int t = 16 * wave + 4 * (l16 & 3) + g;
+            const bool isq = l16 < 4, valid = t < Cn;
+            const float inv = 1.0f / sqrtf(mine + p.eps);
+            (isq ? qi : ki)[t] = !valid ? 0.0f : !p.l2norm ? 1.0f : isq ? inv * inv_scale_q : inv;
+            if (valid && !is_finite_f(mine)) bad = 1;
         }
     } else {
         // 1. normalised rows (as math.rs:833-846) and the norms for the row scales:
@@ -424,6 +435,8 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
         acc[u] = a4;
     }
     __syncthreads();  // every read of the rows is done: A goes over them
+    // non-finite values seen: x * 0 is NaN for an infinity or a NaN, else 0
+    float nf = 0.0f;
 #pragma unroll
     for (int u = 0; u < 5; u++) {
         const int ti = wave + 4 * u;
@@ -431,18 +444,20 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
         const int r = tt < 1 ? 0 : tt < 3 ? 1 : tt < 6 ? 2 : 3;
         const int q = tt - r * (r + 1) / 2;
         const int s = 16 * q + l16;
+        const float ks = RAW ? ki[s] : 1.0f;
+        const double ls = lg[s];
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int tl = 4 * g + i;
             const int t = 16 * r + tl;
-            const float dec = s <= t ? expf((float)(lg[t] - lg[s])) : 0.0f;
+            const float dec = expf((float)(lg[t] - ls));  // (used for s <= t only)
             if (ti < kTpTiles) {
-                const float gr = RAW ? ki[t] * ki[s] * acc[u][i] : acc[u][i];
+                const float gr = RAW ? ki[t] * ks * acc[u][i] : acc[u][i];
                 am[t * AMS + s] = s < t ? bt[t] * dec * gr : 0.0f;
             } else {
-                const float pr = RAW ? qi[t] * ki[s] * acc[u][i] : acc[u][i];
+                const float pr = RAW ? qi[t] * ks * acc[u][i] : acc[u][i];
                 const float v = s <= t ? dec * pr : 0.0f;
-                if (!is_finite_f(v)) bad = 1;
+                nf = fmaf(v, 0.0f, nf);
                 *(float*)(blk + (BF ? kBfP : kTpP) + tt * 1024 + 4 * tp_elem(tl, l16)) = v;
             }
         }
@@ -470,7 +485,7 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
         }
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-            if (!is_finite_f(x[e])) bad = 1;
+            nf = fmaf(x[e], 0.0f, nf);
             tm[(16 * wave + 4 * part + e) * AMS + 16 * wave + col] = x[e];
             if constexpr (!BF) *(float*)(blk + kTpT + tp_tri(wave, wave) * 1024 + 4 * tp_elem(4 * part + e, col)) = x[e];
         }
@@ -501,7 +516,7 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
             tb[n] = -(z0 + z1);
 #pragma unroll
             for (int e = 0; e < 4; e++) {
-                if (!is_finite_f(tb[n][e])) bad = 1;
+                nf = fmaf(tb[n][e], 0.0f, nf);
                 if constexpr (BF) tm[(16 * i + 4 * g + e) * AMS + 16 * wave + l16] = tb[n][e];
                 else *(float*)(blk + kTpT + tp_tri(i, wave) * 1024 + 4 * tp_elem(4 * g + e, l16)) = tb[n][e];
             }
@@ -528,6 +543,7 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
                     make_uint4(lo[pc].x, lo[pc].y, hi[pc].x, hi[pc].y);
         }
     }
+    if (nf != 0.0f) bad = 1;
     // 4. row scales, gamma_last, flag
     if (tid < C) {
         const int t = tid;
