@@ -124,7 +124,8 @@ uint32_t next_f16_epoch() {
 
 // in_dtype: element type of a->q / a->k / a->v (the public entry point uses
 // a->dtype; the run-state path stages the reference's f32 rows directly).
-int prefill_enqueue_ex(const gr_prefill_args* a, int in_dtype, hipStream_t st) {
+// feed: the run-state path's rows still on their way (null: all there).
+int prefill_enqueue_ex(const gr_prefill_args* a, int in_dtype, hipStream_t st, const PrepFeed* feed) {
     int rc = check_prefill(a);
     if (rc) return rc;
     if (a->n_tokens == 0) return GR_OK;
@@ -207,7 +208,7 @@ int prefill_enqueue_ex(const gr_prefill_args* a, int in_dtype, hipStream_t st) {
         e = launch_bf16_rows_to_f16(hc, st);
         if (e != hipSuccess) return hip_fail(e, "gr_prefill_attention bf16 copy launch");
     }
-    e = launch_qkv_prep(pp, st);
+    e = launch_qkv_prep_fed(pp, feed, st);
     if (e != hipSuccess) return hip_fail(e, "gr_prefill_attention prep launch");
 
     PrefillLaunch pf{};
@@ -278,7 +279,7 @@ size_t gr_prefill_workspace_size(const gr_prefill_args* a) { return gr::prefill_
 
 int gr_prefill_attention(const gr_prefill_args* a, void* stream) {
     gr::clear_error();
-    return gr::prefill_enqueue_ex(a, a ? a->dtype : 0, (hipStream_t)stream);
+    return gr::prefill_enqueue_ex(a, a ? a->dtype : 0, (hipStream_t)stream, nullptr);
 }
 
 int gr_rope_freqs(float theta, int32_t rope_dim, float* freqs_out) {

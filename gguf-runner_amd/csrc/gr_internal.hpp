@@ -4,6 +4,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <functional>
+#include <vector>
+
 #include "prefill_split.hpp"
 
 namespace gr {
@@ -151,6 +154,15 @@ struct QkvPrepLaunch {
 };
 
 hipError_t launch_qkv_prep(const QkvPrepLaunch& p, hipStream_t st);
+
+// The prep pass of rows that the host is still copying to where the kernels read them:
+// tokens [cut[i], cut[i + 1]) are launched as soon as fill(i) has put them there, so
+// the host copies piece i + 1 while the GPU reads piece i.
+struct PrepFeed {
+    std::vector<int> cut;
+    std::function<void(int)> fill;
+};
+hipError_t launch_qkv_prep_fed(const QkvPrepLaunch& p, const PrepFeed* feed, hipStream_t st);
 
 // f16 copies of cache rows [row0, row0 + n_rows) of a bf16 K and V cache (row
 // stride cache_row_stride elements, kv_dim elements per row) into rows 0.. of

@@ -300,4 +300,36 @@ hipError_t launch_qkv_prep(const QkvPrepLaunch& p, hipStream_t st) {
     return p.n_tokens >= kPrepWaveTokens ? launch_qkv_prep_t<kPrepRowsPerBlock>(p, st) : launch_qkv_prep_t<1>(p, st);
 }
 
+hipError_t launch_qkv_prep_fed(const QkvPrepLaunch& p, const PrepFeed* feed, hipStream_t st) {
+    if (!feed) return launch_qkv_prep(p, st);
+    auto at = [](const void* x, int64_t elems, int dt) {
+        return x ? (void*)((char*)x + elems * (dt == GR_DTYPE_F32 ? 4 : 2)) : nullptr;
+    };
+    for (size_t i = 0; i + 1 < feed->cut.size(); i++) {
+        feed->fill((int)i);
+        const int64_t r0 = feed->cut[i];
+        const int64_t qo = r0 * p.n_heads * p.head_dim;
+        QkvPrepLaunch c = p;
+        c.n_tokens = feed->cut[i + 1] - (int)r0;
+        if (p.pos) c.pos = p.pos + r0;
+        c.pos0 = p.pos0 + r0;
+        c.q = at(p.q, r0 * p.q_row_stride, p.in_dtype);
+        c.k = at(p.k, r0 * p.kv_row_stride, p.in_dtype);
+        c.v = at(p.v, r0 * p.kv_row_stride, p.in_dtype);
+        c.q_out = at(p.q_out, qo, p.q_out_dtype);
+        c.q_out_lo = at(p.q_out_lo, qo, p.q_out_dtype);
+        if (p.cache_by_index) {
+            c.k_cache = at(p.k_cache, r0 * p.cache_row_stride, p.cache_dtype);
+            c.v_cache = at(p.v_cache, r0 * p.cache_row_stride, p.cache_dtype);
+        }
+        if (p.cache_row) c.cache_row = p.cache_row + r0;
+        if (p.cache_seq) c.cache_seq = p.cache_seq + r0;
+        if (p.rope_cs_out) c.rope_cs_out = p.rope_cs_out + r0 * p.rope_dim;
+        if (i > 0) c.n_copy = 0;
+        const hipError_t e = launch_qkv_prep(c, st);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 }  // namespace gr
