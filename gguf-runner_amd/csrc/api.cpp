@@ -260,11 +260,11 @@ int decode_enqueue(const gr_decode_args* a, hipStream_t st) { return decode_enqu
 
 // seq_slot: optional device map from batch entry to cache sequence slot.
 int decode_enqueue_ex(const gr_decode_args* a, const int32_t* seq_slot, hipStream_t st) {
-    return decode_enqueue_ex(a, seq_slot, st, 0, nullptr, nullptr);
+    return decode_enqueue_ex(a, seq_slot, st, 0, nullptr, nullptr, nullptr);
 }
 
 int decode_enqueue_ex(const gr_decode_args* a, const int32_t* seq_slot, hipStream_t st, int tok_pack,
-                      const int32_t* col_start, const int32_t* col_end) {
+                      const int32_t* col_start, const int32_t* col_end, const TurboToken* token) {
     int rc = check_decode(a);
     if (rc) return rc;
     if (tok_pack > 0 && (a->kv_dtype != GR_DTYPE_TURBO || seq_slot || !col_start || !col_end || a->split_keys <= 0 ||
@@ -322,6 +322,7 @@ int decode_enqueue_ex(const gr_decode_args* a, const int32_t* seq_slot, hipStrea
         p.tok_pack = tok_pack;
         p.col_start = col_start;
         p.col_end = col_end;
+        p.token = token;
     }
     hipError_t e = launch_decode(p, st);
     if (e != hipSuccess) return hip_fail(e, "gr_decode_attention launch");

@@ -187,7 +187,10 @@ size_t q8_stage_bytes(const gr_run_state* s, size_t n) {
 // the caller, sequence slot `seq` already folded into them unless p.cache_seq is
 // given).  Q8: the prep kernel writes f32 rows to staging and the Q8 write
 // kernel quantises them into the cache rows (kv_write_token, inference.rs:1886-1917).
-int prep_and_store(gr_run_state* s, int l, int seq, QkvPrepLaunch p, Carve& cv, const PrepFeed* feed = nullptr) {
+// Turbo, with `token`: a few tokens' passes are left to the decode's first launch
+// (token->set).
+int prep_and_store(gr_run_state* s, int l, int seq, QkvPrepLaunch p, Carve& cv, const PrepFeed* feed = nullptr,
+                   TurboToken* token = nullptr) {
     hipError_t e;
     if (!is_q8(s) && !is_turbo(s)) {
         e = launch_qkv_prep_fed(p, feed, s->stream);
@@ -222,6 +225,13 @@ int prep_and_store(gr_run_state* s, int l, int seq, QkvPrepLaunch p, Carve& cv, 
         w.cache_row = p.cache_row ? p.cache_row : p.pos;
         w.cache_seq = p.cache_seq;
         w.row0 = p.pos0;
+        if (token && (int64_t)p.n_tokens * (p.n_heads + 2 * p.n_kv_heads) <= kTurboTokenRows) {
+            token->prep = p;
+            token->write = w;
+            token->feed = feed;
+            token->set = true;
+            return GR_OK;
+        }
         p.k_cache = kst;
         p.v_cache = vst;
         p.cache_dtype = GR_DTYPE_F32;
@@ -614,7 +624,9 @@ static gr_decode_args turbo_pack_probe(const gr_run_state* s, int n, const Turbo
 // device; null: uploaded here on the state's stream.
 static int run_decode(gr_run_state* s, int layer, int n, const float* qdev, const int32_t* slots_dev, int seq,
                       const std::vector<int32_t>& starts, const std::vector<int32_t>& ends, float* xb_dev,
-                      Carve& cv, const TurboPack* pack = nullptr, const int32_t* se_dev = nullptr) {
+                      Carve& cv, const TurboPack* pack = nullptr, const int32_t* se_dev = nullptr,
+                      const TurboToken* token = nullptr) {
+    if (token && !token->set) token = nullptr;
     std::vector<int32_t> host(2 * (size_t)n);
     int max_len = 1;
     for (int b = 0; b < n; b++) {
@@ -675,8 +687,9 @@ static int run_decode(gr_run_state* s, int layer, int n, const float* qdev, cons
     }
     const size_t ws = decode_ws_bytes(&a);
     a.workspace = cv.take<char>(ws + 256);
-    if (pack) return decode_enqueue_ex(&a, slots_dev, s->stream, pack->tp, se + 2 * (size_t)n, se + 3 * (size_t)n);
-    return decode_enqueue_ex(&a, slots_dev, s->stream);
+    if (pack)
+        return decode_enqueue_ex(&a, slots_dev, s->stream, pack->tp, se + 2 * (size_t)n, se + 3 * (size_t)n, token);
+    return decode_enqueue_ex(&a, slots_dev, s->stream, 0, nullptr, nullptr, token);
 }
 
 int gr_attention_token(gr_run_state* s, int32_t seq, int32_t layer, int64_t pos, const float* q, float* xb) {
@@ -753,8 +766,9 @@ int gr_attention_layer_token(gr_run_state* s, int32_t seq, int32_t layer, int64_
     p.q_out = qp;
     p.k_cache = (char*)layer_k(s, layer) + cache_bytes_at(s, (size_t)seq * s->seq_stride);
     p.v_cache = (char*)layer_v(s, layer) + cache_bytes_at(s, (size_t)seq * s->seq_stride);
-    if ((rc = prep_and_store(s, layer, seq, p, cv))) return rc;
-    if ((rc = run_decode(s, layer, 1, qp, nullptr, seq, {st}, {en}, xo, cv, nullptr, se_dev))) return rc;
+    TurboToken token;
+    if ((rc = prep_and_store(s, layer, seq, p, cv, nullptr, &token))) return rc;
+    if ((rc = run_decode(s, layer, 1, qp, nullptr, seq, {st}, {en}, xo, cv, nullptr, se_dev, &token))) return rc;
     return mp ? mr.finish() : d2h_sync(s, xb, xo, qb);
 }
 
@@ -983,7 +997,8 @@ static int prefill_rows(gr_run_state* s, int32_t seq, int32_t layer, int64_t bas
             p.copy_dst = se_dev[pc];
             p.n_copy = (int)se[pc].size();
         }
-        int r = prep_and_store(s, layer, seq, p, cw, fp);
+        TurboToken token;
+        int r = prep_and_store(s, layer, seq, p, cw, fp, &token);
         if (r) return r;
         if (is_q8(s)) {
             // one MFMA flash pass over the int8 rows (all n queries share each K / V tile)
@@ -1012,7 +1027,7 @@ static int prefill_rows(gr_run_state* s, int32_t seq, int32_t layer, int64_t bas
             return e == hipSuccess ? GR_OK : hip_fail(e, "q8 prefill launch");
         }
         return run_decode(s, layer, n, qp, nullptr, seq, pst[pc], pen[pc], xi, cw,
-                          packs[pc].tp > 0 ? &packs[pc] : nullptr, se_dev[pc]);
+                          packs[pc].tp > 0 ? &packs[pc] : nullptr, se_dev[pc], &token);
     };
 
     if (mp) {
@@ -1120,8 +1135,9 @@ int gr_decode_layer_batch(gr_run_state* s, int32_t layer, int32_t n, const int32
     p.v_cache = layer_v(s, layer);
     p.cache_seq = mp ? sse_host : slot_d;  // the prep's own reads: the device copy is not there yet
     p.cache_seq_stride = (int64_t)s->seq_stride;
-    if ((rc = prep_and_store(s, layer, 0, p, cv))) return rc;
-    if ((rc = run_decode(s, layer, n, qp, slot_d, 0, starts, ends, xo, cv, nullptr, se_dev))) return rc;
+    TurboToken token;
+    if ((rc = prep_and_store(s, layer, 0, p, cv, nullptr, &token))) return rc;
+    if ((rc = run_decode(s, layer, n, qp, slot_d, 0, starts, ends, xo, cv, nullptr, se_dev, &token))) return rc;
     return mp ? mr.finish() : d2h_sync(s, xb, xo, qb);
 }
 

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "gr_attn.h"
+
 #include <functional>
 #include <vector>
 
@@ -26,6 +28,8 @@ struct OutGate {
 
 // Sequences per launch on the stream schedule (per-workgroup LDS tables).
 constexpr int kStreamMaxSeq = 1024;
+
+struct TurboToken;
 
 struct DecodeLaunch {
     int n_seq, n_heads, n_kv_heads, head_dim, kv_dtype;
@@ -91,6 +95,9 @@ struct DecodeLaunch {
     // grid is KV head vg / n_sub with query heads (vg / n_sub) * kv_mul + (vg % n_sub)
     // * sub_heads .. + min(sub_heads, kv_mul - (vg % n_sub) * sub_heads).  0 = 1.
     int n_sub = 0, sub_heads = 0;
+    // Turbo, run state: the tokens' rows are prepared, written and rotated by one launch
+    // ahead of the split kernel (host pointer; q is not read); null: q is there.
+    const TurboToken* token = nullptr;
 };
 
 hipError_t launch_decode(const DecodeLaunch& p, hipStream_t st);
@@ -164,6 +171,40 @@ struct PrepFeed {
 };
 hipError_t launch_qkv_prep_fed(const QkvPrepLaunch& p, const PrepFeed* feed, hipStream_t st);
 
+// launch(piece, first token) for the pieces of a fed prep (null feed: p itself).
+template <typename F>
+hipError_t for_prep_pieces(const QkvPrepLaunch& p, const PrepFeed* feed, F launch) {
+    if (!feed) return launch(p, 0);
+    auto at = [](const void* x, int64_t elems, int dt) {
+        return x ? (void*)((char*)x + elems * (dt == GR_DTYPE_F32 ? 4 : 2)) : nullptr;
+    };
+    for (size_t i = 0; i + 1 < feed->cut.size(); i++) {
+        feed->fill((int)i);
+        const int64_t r0 = feed->cut[i];
+        const int64_t qo = r0 * p.n_heads * p.head_dim;
+        QkvPrepLaunch c = p;
+        c.n_tokens = feed->cut[i + 1] - (int)r0;
+        if (p.pos) c.pos = p.pos + r0;
+        c.pos0 = p.pos0 + r0;
+        c.q = at(p.q, r0 * p.q_row_stride, p.in_dtype);
+        c.k = at(p.k, r0 * p.kv_row_stride, p.in_dtype);
+        c.v = at(p.v, r0 * p.kv_row_stride, p.in_dtype);
+        c.q_out = at(p.q_out, qo, p.q_out_dtype);
+        c.q_out_lo = at(p.q_out_lo, qo, p.q_out_dtype);
+        if (p.cache_by_index) {
+            c.k_cache = at(p.k_cache, r0 * p.cache_row_stride, p.cache_dtype);
+            c.v_cache = at(p.v_cache, r0 * p.cache_row_stride, p.cache_dtype);
+        }
+        if (p.cache_row) c.cache_row = p.cache_row + r0;
+        if (p.cache_seq) c.cache_seq = p.cache_seq + r0;
+        if (p.rope_cs_out) c.rope_cs_out = p.rope_cs_out + r0 * p.rope_dim;
+        if (i > 0) c.n_copy = 0;
+        const hipError_t e = launch(c, (int)r0);
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 // f16 copies of cache rows [row0, row0 + n_rows) of a bf16 K and V cache (row
 // stride cache_row_stride elements, kv_dim elements per row) into rows 0.. of
 // k_f16 / v_f16 (row stride kv_dim), with the range flag of QkvPrepLaunch.
@@ -231,6 +272,18 @@ struct TurboWriteLaunch {
 };
 
 hipError_t launch_turbo_write(const TurboWriteLaunch& p, hipStream_t st);
+
+// A few tokens' preparation, Turbo write and query preparation in one launch ahead of
+// the split kernel (DecodeLaunch::token): prep's q_out / k_cache / v_cache and write's
+// k_rows / v_rows are not used.  From kTurboTokenRows head rows on the passes of their
+// own are used (their waves take several rows each).
+struct TurboToken {
+    QkvPrepLaunch prep{};
+    TurboWriteLaunch write{};
+    const PrepFeed* feed = nullptr;
+    bool set = false;  // filled in
+};
+constexpr int kTurboTokenRows = 3072;
 
 // Qwen3.5 SSM layer pre/post around the DeltaNet recurrence for a chunk of
 // n_tokens tokens.  qkv [T][conv_dim] (conv_dim = (n_v + 2 n_k) head_dim),

@@ -11,24 +11,12 @@
 
 #include "gr_common.hpp"
 #include "gr_internal.hpp"
+#include "qkv_row.hpp"
 
 namespace gr {
 
 constexpr int kPrepThreads = 256;
 constexpr int kPrepRowsPerBlock = kPrepThreads / 64;
-
-// 8 consecutive elements (one 16-byte chunk of a 16-bit row, two of an f32 row).
-__device__ __forceinline__ void load8(const void* base, size_t idx, int dt, float* v) {
-    if (dt == GR_DTYPE_F32) {
-        const float4 a = *(const float4*)((const float*)base + idx);
-        const float4 b = *(const float4*)((const float*)base + idx + 4);
-        v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
-        return;
-    }
-    const uint4 u = *(const uint4*)((const uint16_t*)base + idx);
-    if (dt == GR_DTYPE_F16) unpack16<F16>(u, v);
-    else unpack16<BF16>(u, v);
-}
 
 __device__ __forceinline__ void store8(void* base, size_t idx, int dt, const float* v) {
     if (dt == GR_DTYPE_F32) {
@@ -74,19 +62,10 @@ __global__ __launch_bounds__(kPrepThreads) void qkv_prep_kernel(const QkvPrepLau
         for (int t = threadIdx.x; t < p.n_copy; t += kPrepThreads) p.copy_dst[t] = p.copy_src[t];
     const int rows_per_token = p.n_heads + 2 * p.n_kv_heads;
     const int64_t pos = p.pos ? (int64_t)p.pos[i] : p.pos0 + i;
-    const bool rope = p.rope_mode != GR_ROPE_NONE;
     const int half = p.rope_dim / 2;
-    if (rope) {
-        for (int f = wt * 64 + lane; f < half; f += WPT * 64) {
-            const float val = ((float)pos * p.rope_freqs[f]) * p.rope_scale;
-            float sn, cs;
-            sincosf(val, &sn, &cs);
-            cs_t[f] = cs;
-            sn_t[f] = sn;
-            if (p.rope_cs_out && tok_ok && blockIdx.y == 0)
-                *(float2*)(p.rope_cs_out + ((size_t)i * half + f) * 2) = make_float2(cs, sn);
-        }
-    }
+    if (p.rope_mode != GR_ROPE_NONE)
+        prep_rope_table(p, pos, wt * 64 + lane, WPT * 64, cs_t, sn_t,
+                        p.rope_cs_out && tok_ok && blockIdx.y == 0 ? p.rope_cs_out + (size_t)i * half * 2 : nullptr);
     __syncthreads();
     if (!tok_ok) return;  // no workgroup barrier below
     float* rb = row_buf[wave][rsub];
@@ -105,89 +84,8 @@ __global__ __launch_bounds__(kPrepThreads) void qkv_prep_kernel(const QkvPrepLau
         const int kind = hrc < p.n_heads ? 0 : (hrc < p.n_heads + p.n_kv_heads ? 1 : 2);  // q, k, v
         const int head = kind == 0 ? hrc : (kind == 1 ? hrc - p.n_heads : hrc - p.n_heads - p.n_kv_heads);
         const bool skip = !valid || (kind == 0 && p.q_out == nullptr);
-        const void* src = kind == 0 ? p.q : (kind == 1 ? p.k : p.v);
-        const int64_t rs = kind == 0 ? p.q_row_stride : p.kv_row_stride;
         float x[8];
-        if (!skip) load8(src, (size_t)i * rs + (size_t)head * D + c8, p.in_dtype, x);
-        else
-#pragma unroll
-            for (int e = 0; e < 8; e++) x[e] = 0.0f;
-        // Qwen2 attention biases, before the norm (qkv_bias_and_norm, inference.rs:2545-2559)
-        const float* bias = kind == 0 ? p.q_bias : (kind == 1 ? p.k_bias : p.v_bias);
-        if (bias && !skip) {
-            float bv[8];
-            load8(bias, (size_t)head * D + c8, GR_DTYPE_F32, bv);
-#pragma unroll
-            for (int e = 0; e < 8; e++) x[e] += bv[e];
-        }
-        if (kind != 2) {
-            // QK RMSNorm: ss = sum(x^2)/d + eps; x = w * ((1/sqrt(ss)) * x).
-            const float* w = kind == 0 ? p.q_norm : p.k_norm;
-            float ss = 0.0f;
-#pragma unroll
-            for (int e = 0; e < 8; e++) ss += x[e] * x[e];
-            ss = wave_sum<LPR>(ss);  // lanes of other rows never mix: groups are LPR-aligned
-            if (w) {
-                const float inv = 1.0f / sqrtf(ss / (float)D + p.eps);
-                float wv[8];
-                load8(w, c8, GR_DTYPE_F32, wv);
-#pragma unroll
-                for (int e = 0; e < 8; e++) x[e] = wv[e] * (inv * x[e]);
-            }
-            if (rope) {
-                if (p.rope_mode == GR_ROPE_ADJACENT) {
-                    // pairs (2j, 2j+1) sit inside the lane's 8 elements
-#pragma unroll
-                    for (int e = 0; e < 8; e += 2) {
-                        const int fi = (c8 + e) >> 1;
-                        const float cs = cs_t[fi], sn = sn_t[fi];
-                        const float v0 = x[e], v1 = x[e + 1];
-                        x[e] = v0 * cs - v1 * sn;
-                        x[e + 1] = v0 * sn + v1 * cs;
-                    }
-                } else if (p.rope_dim == D) {
-                    // NeoX pairs (i, i + D/2) of a fully rotated row: the partner
-                    // elements of this lane's 8 are the 8 of lane ^ (LPR/2), in the
-                    // same row's lane group
-                    const bool first = c8 < half;
-                    const int f0 = first ? c8 : c8 - half;
-                    float csv[8], snv[8];
-                    *(float4*)csv = *(const float4*)(cs_t + f0);
-                    *(float4*)(csv + 4) = *(const float4*)(cs_t + f0 + 4);
-                    *(float4*)snv = *(const float4*)(sn_t + f0);
-                    *(float4*)(snv + 4) = *(const float4*)(sn_t + f0 + 4);
-#pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        const float other = __shfl_xor(x[e], LPR / 2, 64);
-                        // (v0, v1) -> (v0*c - v1*s, v0*s + v1*c)
-                        x[e] = first ? x[e] * csv[e] - other * snv[e] : other * snv[e] + x[e] * csv[e];
-                    }
-                } else {
-                    // NeoX pairs (i, i + rope_dim/2) of a partial rotation live in
-                    // other lanes: stage the row
-#pragma unroll
-                    for (int e = 0; e < 8; e++) rb[c8 + e] = x[e];
-                    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        const int idx = c8 + e;
-                        if (idx >= p.rope_dim) continue;  // partial RoPE: tail untouched
-                        const bool first = idx < half;
-                        const int fi = first ? idx : idx - half;
-                        const float other = rb[first ? idx + half : idx - half];
-                        const float cs = cs_t[fi], sn = sn_t[fi];
-                        // (v0, v1) -> (v0*c - v1*s, v0*s + v1*c)
-                        x[e] = first ? x[e] * cs - other * sn : other * sn + x[e] * cs;
-                    }
-                    __builtin_amdgcn_wave_barrier();  // reads done before the next rows' stores
-                }
-            }
-            if (kind == 0 && p.gemma_q_scale) {
-                const float sc = 1.0f / sqrtf((float)D);
-#pragma unroll
-                for (int e = 0; e < 8; e++) x[e] *= sc;
-            }
-        }
+        prep_row<D>(p, i, kind, head, skip, c8, cs_t, sn_t, rb, x);
         if (skip) continue;
         if (kind == 0) {
             const size_t ob = ((size_t)i * p.n_heads + head) * D + c8;
@@ -301,35 +199,7 @@ hipError_t launch_qkv_prep(const QkvPrepLaunch& p, hipStream_t st) {
 }
 
 hipError_t launch_qkv_prep_fed(const QkvPrepLaunch& p, const PrepFeed* feed, hipStream_t st) {
-    if (!feed) return launch_qkv_prep(p, st);
-    auto at = [](const void* x, int64_t elems, int dt) {
-        return x ? (void*)((char*)x + elems * (dt == GR_DTYPE_F32 ? 4 : 2)) : nullptr;
-    };
-    for (size_t i = 0; i + 1 < feed->cut.size(); i++) {
-        feed->fill((int)i);
-        const int64_t r0 = feed->cut[i];
-        const int64_t qo = r0 * p.n_heads * p.head_dim;
-        QkvPrepLaunch c = p;
-        c.n_tokens = feed->cut[i + 1] - (int)r0;
-        if (p.pos) c.pos = p.pos + r0;
-        c.pos0 = p.pos0 + r0;
-        c.q = at(p.q, r0 * p.q_row_stride, p.in_dtype);
-        c.k = at(p.k, r0 * p.kv_row_stride, p.in_dtype);
-        c.v = at(p.v, r0 * p.kv_row_stride, p.in_dtype);
-        c.q_out = at(p.q_out, qo, p.q_out_dtype);
-        c.q_out_lo = at(p.q_out_lo, qo, p.q_out_dtype);
-        if (p.cache_by_index) {
-            c.k_cache = at(p.k_cache, r0 * p.cache_row_stride, p.cache_dtype);
-            c.v_cache = at(p.v_cache, r0 * p.cache_row_stride, p.cache_dtype);
-        }
-        if (p.cache_row) c.cache_row = p.cache_row + r0;
-        if (p.cache_seq) c.cache_seq = p.cache_seq + r0;
-        if (p.rope_cs_out) c.rope_cs_out = p.rope_cs_out + r0 * p.rope_dim;
-        if (i > 0) c.n_copy = 0;
-        const hipError_t e = launch_qkv_prep(c, st);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
+    return for_prep_pieces(p, feed, [&](const QkvPrepLaunch& c, int) { return launch_qkv_prep(c, st); });
 }
 
 }  // namespace gr

@@ -22,35 +22,9 @@
 #include "gr_internal.hpp"
 #include "stream_sched.hpp"
 #include "turbo_common.hpp"
+#include "turbo_write.hpp"
 
 namespace gr {
-
-namespace {
-
-__device__ __forceinline__ float tq_centroid(int code) {
-    return code == 0 ? -tq::kC1 : code == 1 ? -tq::kC0 : code == 2 ? tq::kC0 : tq::kC1;
-}
-
-__device__ __forceinline__ int tq_code(float x) {
-    return x < -tq::kTh ? 0 : (x < 0.0f ? 1 : (x < tq::kTh ? 2 : 3));
-}
-
-// l2_norm (math.rs:467-473): sequential sum in element order, every lane the same
-template <int D>
-__device__ __forceinline__ float wave_l2_sequential(const float (&x)[D / 64], float* buf, int lane) {
-#pragma unroll
-    for (int j = 0; j < D / 64; j++) buf[lane + 64 * j] = x[j];
-    __syncthreads();  // one-wave workgroup
-    float ss = 0.0f;
-    for (int e = 0; e < D; e++) {
-        const float v = buf[e];
-        ss = ss + v * v;
-    }
-    __syncthreads();  // buf is reused by the caller
-    return sqrtf(ss);
-}
-
-}  // namespace
 
 // ---------------------------------------------------------------- KV write
 
@@ -64,61 +38,11 @@ __global__ __launch_bounds__(64) void turbo_write_kernel(const TurboWriteLaunch 
     const int lane = threadIdx.x;
     const int i = blockIdx.x, g = blockIdx.y;
     const bool is_v = blockIdx.z != 0;
-    const int kv_dim = p.n_kv_heads * D;
-    const float* src = (is_v ? p.v_rows : p.k_rows) + (size_t)i * kv_dim + (size_t)g * D;
-    const int64_t row = p.cache_row ? (int64_t)p.cache_row[i] : p.row0 + i;
-    const int64_t sq = p.cache_seq ? (int64_t)p.cache_seq[i] : 0;
-    const int64_t elem = sq * p.cache_seq_stride + row * p.cache_row_stride + (int64_t)g * D;
-    uint8_t* base = (is_v ? p.v_base : p.k_base) + elem / 4;
-    uint8_t* sign = (is_v ? p.v_sign : p.k_sign) + elem / 8;
-    const int64_t aux = sq * p.aux_seq_stride + row * p.aux_row_stride + g;
-    float* scale_out = (is_v ? p.v_scale : p.k_scale) + aux;
-    float* rnorm_out = (is_v ? p.v_rnorm : p.k_rnorm) + aux;
-    const uint8_t* sg = p.signs + (size_t)g * (D / 8);
-    const int64_t ss = p.slot_stride;
-
+    const float* src = (is_v ? p.v_rows : p.k_rows) + ((size_t)i * p.n_kv_heads + g) * D;
     float x[J];
 #pragma unroll
     for (int j = 0; j < J; j++) x[j] = src[lane + 64 * j];
-    tq::wave_transform<D>(x, sg, sg + ss, lane);  // rot_pre, rot_post
-    const float sigma = wave_l2_sequential<D>(x, buf, lane) / sqrtf((float)D);
-    if (sigma == 0.0f) {
-        if (lane == 0) {
-            *scale_out = 0.0f;
-            *rnorm_out = 0.0f;
-        }
-        if (lane < D / 4) base[lane] = 0;
-        if (lane < D / 8) sign[lane] = 0xff;
-        return;
-    }
-    const float inv_sigma = 1.0f / sigma;
-    float r[J];
-#pragma unroll
-    for (int j = 0; j < J; j++) {
-        const int c = tq_code(x[j] * inv_sigma);
-        r[j] = x[j] - tq_centroid(c) * sigma;
-        codes[lane + 64 * j] = (uint8_t)c;
-    }
-    const float gamma = wave_l2_sequential<D>(r, buf, lane);  // its barrier also publishes `codes`
-    if (lane < D / 4)
-        base[lane] = (uint8_t)(codes[4 * lane] | (codes[4 * lane + 1] << 2) | (codes[4 * lane + 2] << 4) |
-                               (codes[4 * lane + 3] << 6));
-    if (lane == 0) {
-        *scale_out = sigma;
-        *rnorm_out = gamma;
-    }
-    if (gamma == 0.0f) {
-        if (lane < D / 8) sign[lane] = 0xff;
-        return;
-    }
-#pragma unroll
-    for (int j = 0; j < J; j++) r[j] = r[j] / gamma;
-    tq::wave_transform<D>(r, sg + 2 * ss, sg + 3 * ss, lane);  // res_pre, res_post
-#pragma unroll
-    for (int j = 0; j < J; j++) {
-        const uint64_t m = __ballot(r[j] >= 0.0f);  // bit l = element 64 j + l
-        if (lane == 0) *(uint64_t*)(sign + 8 * j) = m;
-    }
+    turbo_write_unit<D>(p, i, g, is_v, x, buf, codes, lane);
 }
 
 // The same write for long row sets (a prefill chunk): one wave quantises R
@@ -306,18 +230,23 @@ hipError_t launch_turbo_write(const TurboWriteLaunch& p, hipStream_t st) {
 
 // ---------------------------------------------------------------- merge + finalize
 
-// One wave per (head, sequence): merge the split partials of the base and residual
+// WPH waves per (head, sequence): merge the split partials of the base and residual
 // accumulators (log2-domain weights), divide by the softmax sum, then
 // finalize_turboquant_value_head (inference.rs:1323-1334): residual <- R'^-1
-// residual, base += residual, out = R^-1 base.
-template <int D>
+// residual, base += residual, out = R^-1 base.  Bound by the round trips of the
+// partials' loads: with one wave per head they follow each other eight at a time, so
+// heads of many partials are taken by the workgroup's four waves, a quarter of the
+// partials each (launch_turbo_combine's rule).
+template <int D, int WPH>
 __global__ __launch_bounds__(256) void turbo_combine_kernel(const DecodeLaunch p) {
+    static_assert(WPH == 1 || WPH == 4, "a wave or the workgroup per head");
     constexpr int J = D / 64, U = 8;
     __shared__ float wsh_all[4][64];
+    __shared__ float part[WPH > 1 ? 3 : 1][2 * J + 1][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float* wsh = wsh_all[wave];
-    const int h = 4 * blockIdx.x + wave, s = blockIdx.y;  // four heads per workgroup
-    if (h >= p.n_heads) return;  // whole wave; only wave-level synchronisation below
+    const int h = WPH > 1 ? (int)blockIdx.x : 4 * (int)blockIdx.x + wave, s = blockIdx.y;
+    if (h >= p.n_heads) return;  // the whole wave; WPH 1: only wave-level synchronisation below
     const int kv_mul = p.n_heads / p.n_kv_heads;
     const int g = h / kv_mul;
     const int t_len = p.kv_end[s] - p.kv_start[s];
@@ -336,8 +265,11 @@ __global__ __launch_bounds__(256) void turbo_combine_kernel(const DecodeLaunch p
     float b[J], r[J];
 #pragma unroll
     for (int j = 0; j < J; j++) b[j] = r[j] = 0.0f;
-    for (int c0 = 0; c0 < n_used; c0 += 64) {
-        const int nc = min(64, n_used - c0);
+    // this wave's partials: [p_lo, p_hi)
+    const int per = (n_used + WPH - 1) / WPH;
+    const int p_lo = WPH > 1 ? min(wave * per, n_used) : 0, p_hi = WPH > 1 ? min(p_lo + per, n_used) : n_used;
+    for (int c0 = p_lo; c0 < p_hi; c0 += 64) {
+        const int nc = min(64, p_hi - c0);
         // lane i: the weight of split c0 + i
         float w = 0.0f;
         if (lane < nc) {
@@ -375,6 +307,27 @@ __global__ __launch_bounds__(256) void turbo_combine_kernel(const DecodeLaunch p
         tq::wave_lds_sync();  // wsh reads done before the next chunk's stores
     }
     lt = wave_sum<64>(lt);
+    if constexpr (WPH > 1) {  // every wave's sums are relative to the same maximum
+        if (wave > 0) {
+#pragma unroll
+            for (int j = 0; j < J; j++) {
+                part[wave - 1][2 * j][lane] = b[j];
+                part[wave - 1][2 * j + 1][lane] = r[j];
+            }
+            part[wave - 1][2 * J][lane] = lt;
+        }
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int w = 0; w < WPH - 1; w++) {
+#pragma unroll
+            for (int j = 0; j < J; j++) {
+                b[j] += part[w][2 * j][lane];
+                r[j] += part[w][2 * j + 1][lane];
+            }
+            lt += part[w][2 * J][lane];
+        }
+    }
     const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;
 #pragma unroll
     for (int j = 0; j < J; j++) {
@@ -393,15 +346,27 @@ __global__ __launch_bounds__(256) void turbo_combine_kernel(const DecodeLaunch p
     for (int j = 0; j < J; j++) out[lane + 64 * j] = gt ? gate_mul(b[j], gt[lane + 64 * j]) : b[j];
 }
 
+// More than kTurboCombineWide partials per head possible: a workgroup per head.
+// MI355X, us of this kernel: 2 x 32768 keys, 32 / 4 heads (about 32 partials) 7.8 -> 6.2;
+// a call of 1 x 8000 keys 20.8 -> 19.4 (32 / 4 heads), 20.3 -> 18.7 (32 / 8).
+constexpr int kTurboCombineWide = 8;
+
+template <int D>
+static hipError_t launch_turbo_combine_d(const DecodeLaunch& p, hipStream_t st) {
+    if (p.n_splits > kTurboCombineWide)
+        turbo_combine_kernel<D, 4><<<dim3(p.n_heads, p.n_seq), 256, 0, st>>>(p);
+    else
+        turbo_combine_kernel<D, 1><<<dim3((p.n_heads + 3) / 4, p.n_seq), 256, 0, st>>>(p);
+    return hipGetLastError();
+}
+
 hipError_t launch_turbo_combine(const DecodeLaunch& p, hipStream_t st) {
-    const dim3 grid((p.n_heads + 3) / 4, p.n_seq);
     switch (p.head_dim) {
-        case 64: turbo_combine_kernel<64><<<grid, 256, 0, st>>>(p); break;
-        case 128: turbo_combine_kernel<128><<<grid, 256, 0, st>>>(p); break;
-        case 256: turbo_combine_kernel<256><<<grid, 256, 0, st>>>(p); break;
+        case 64: return launch_turbo_combine_d<64>(p, st);
+        case 128: return launch_turbo_combine_d<128>(p, st);
+        case 256: return launch_turbo_combine_d<256>(p, st);
         default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
 
 }  // namespace gr

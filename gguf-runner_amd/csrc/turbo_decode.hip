@@ -26,8 +26,10 @@
 
 #include "gr_common.hpp"
 #include "gr_internal.hpp"
+#include "qkv_row.hpp"
 #include "stream_sched.hpp"
 #include "turbo_common.hpp"
+#include "turbo_write.hpp"
 
 namespace gr {
 
@@ -248,23 +250,15 @@ __device__ __forceinline__ const QSlots<D>& qslots() {
 //      E = E_code for code k-steps, E_sign for sign k-steps (max |value| in [2^13, 2^14))
 //   then 2^-E_code, 2^-E_sign, (alpha + beta) sum_i q_rot_i s, sum_i q_proj_i s.
 template <int D>
-__global__ __launch_bounds__(256) void turbo_query_kernel(const DecodeLaunch p) {
+__device__ __forceinline__ void turbo_query_head(const DecodeLaunch& p, int s, int h, float (&x)[D / 64],
+                                                 float (*qsh)[D], int lane) {
     using S = Tq<D>;
     constexpr int J = D / 64, KS = S::KS, NB = 16 * KS;
-    __shared__ float qsh_all[4][2][D];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    float (*qsh)[D] = qsh_all[wave];
-    const int h = 4 * blockIdx.x + wave, s = blockIdx.y;  // four heads per workgroup
-    if (h >= p.n_heads) return;  // whole wave; no workgroup barrier below
     const int g = h / (p.n_heads / p.n_kv_heads);
     const uint8_t* sg = p.turbo_signs + (size_t)g * (D / 8);
     const int64_t ss = p.turbo_slot_stride;
-    const float* q = p.q + ((size_t)s * p.n_heads + h) * D;
     uint32_t* out = (uint32_t*)p.ws_q + ((size_t)s * p.n_heads + h) * S::QBW;
     const float qs = p.score_scale * kLog2e;
-    float x[J];
-#pragma unroll
-    for (int j = 0; j < J; j++) x[j] = q[lane + 64 * j];
     tq::wave_transform<D>(x, sg, sg + ss, lane);  // rot_pre, rot_post
     float sr = 0.0f;
 #pragma unroll
@@ -325,6 +319,62 @@ __global__ __launch_bounds__(256) void turbo_query_kernel(const DecodeLaunch p) 
         c[2] = (kAlpha + kBeta) * sr;
         c[3] = sp;
     }
+}
+
+template <int D>
+__global__ __launch_bounds__(256) void turbo_query_kernel(const DecodeLaunch p) {
+    constexpr int J = D / 64;
+    __shared__ float qsh_all[4][2][D];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int h = 4 * blockIdx.x + wave, s = blockIdx.y;  // four heads per workgroup
+    if (h >= p.n_heads) return;  // whole wave; no workgroup barrier below
+    const float* q = p.q + ((size_t)s * p.n_heads + h) * D;
+    float x[J];
+#pragma unroll
+    for (int j = 0; j < J; j++) x[j] = q[lane + 64 * j];
+    turbo_query_head<D>(p, s, h, x, qsh_all[wave], lane);
+}
+
+// A few tokens' rows straight from the inputs to the split kernel's operands: one wave
+// per (token, head row) runs the row's preparation (qkv_row.hpp) and then, for a q
+// row, the query preparation above, for a k or v row the quantising write: one
+// launch instead of the prep pass, the write and the query kernel, whose rows went
+// through memory between them.  Bound by launch and PCIe latency (the rows sit in
+// host memory).  MI355X, gr_attention_layer_token over 1023 keys, 16 / 8 heads
+// d128, per call: 41.6 us with three launches, 35.4 with one.
+template <int D>
+__global__ __launch_bounds__(64) void turbo_token_kernel(const TurboToken f, const DecodeLaunch p, int tok0) {
+    constexpr int LPR = D / 8, J = D / 64;
+    __shared__ float row_buf[64 / LPR][D];
+    __shared__ __attribute__((aligned(16))) float cs_t[D / 2], sn_t[D / 2];
+    __shared__ float qsh[2][D];
+    __shared__ uint8_t codes[D];
+    const QkvPrepLaunch& q = f.prep;
+    const int lane = threadIdx.x;
+    const int i = blockIdx.x, hr = blockIdx.y;  // token, row: q heads, k heads, v heads
+    const int kind = hr < q.n_heads ? 0 : (hr < q.n_heads + q.n_kv_heads ? 1 : 2);
+    const int head = kind == 0 ? hr : (kind == 1 ? hr - q.n_heads : hr - q.n_heads - q.n_kv_heads);
+    if (q.n_copy > 0 && i == 0 && hr == 0)
+        for (int t = lane; t < q.n_copy; t += 64) q.copy_dst[t] = q.copy_src[t];
+    const int64_t pos = q.pos ? (int64_t)q.pos[i] : q.pos0 + i;
+    if (q.rope_mode != GR_ROPE_NONE && kind != 2) prep_rope_table(q, pos, lane, 64, cs_t, sn_t, nullptr);
+    tq::wave_lds_sync();
+    // every lane group of D / 8 lanes prepares the same row
+    const int c8 = (lane % LPR) * 8;
+    float x8[8];
+    prep_row<D>(q, i, kind, head, false, c8, cs_t, sn_t, row_buf[lane / LPR], x8);
+    tq::wave_lds_sync();  // (a partial rotation's reads of row_buf precede the stores)
+    if (lane < LPR) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) row_buf[0][c8 + e] = kind == 0 ? x8[e] * q.q_out_scale : x8[e];
+    }
+    tq::wave_lds_sync();
+    float x[J];
+#pragma unroll
+    for (int j = 0; j < J; j++) x[j] = row_buf[0][lane + 64 * j];
+    tq::wave_lds_sync();
+    if (kind == 0) turbo_query_head<D>(p, tok0 + i, head, x, qsh, lane);
+    else turbo_write_unit<D>(f.write, i, head, kind == 2, x, row_buf[0], codes, lane);
 }
 
 // ---------------------------------------------------------------- split kernel
@@ -958,8 +1008,22 @@ static hipError_t launch_turbo_d(const DecodeLaunch& p0, hipStream_t st) {
     DecodeLaunch p = p0;  // decode: groups above 16 query heads in columns of 16
     p.n_sub = p.tok_pack > 0 ? 1 : (p.n_heads / p.n_kv_heads + 15) / 16;
     p.sub_heads = 16;
-    turbo_query_kernel<D><<<dim3((p.n_heads + 3) / 4, p.n_seq), 256, 0, st>>>(p);
-    hipError_t e = hipGetLastError();
+    hipError_t e;
+    if (p.token) {
+        const TurboToken& f = *p.token;
+        TurboToken c = f;
+        e = for_prep_pieces(f.prep, f.feed, [&](const QkvPrepLaunch& prep, int r0) {
+            c.prep = prep;
+            c.write.row0 = f.write.row0 + r0;
+            c.write.cache_row = f.write.cache_row ? f.write.cache_row + r0 : nullptr;
+            c.write.cache_seq = f.write.cache_seq ? f.write.cache_seq + r0 : nullptr;
+            turbo_token_kernel<D><<<dim3(prep.n_tokens, prep.n_heads + 2 * prep.n_kv_heads), 64, 0, st>>>(c, p, r0);
+            return hipGetLastError();
+        });
+    } else {
+        turbo_query_kernel<D><<<dim3((p.n_heads + 3) / 4, p.n_seq), 256, 0, st>>>(p);
+        e = hipGetLastError();
+    }
     if (e != hipSuccess) return e;
     const int kv_mul = p.n_heads / p.n_kv_heads;
     const int n_col = p.tok_pack > 0 ? p.tok_pack * kv_mul : std::min(kv_mul, 16);
