@@ -91,6 +91,23 @@ def test_encoder_attention_matches_oracle(orc, dev, ns, tps, hc, hd, mag):
     assert e_gpu <= e_orc + TOL_STRESS, f"device {e_gpu:.3e} vs oracle {e_orc:.3e} from float64"
 
 
+@pytest.mark.parametrize("ns,tps,hc,hd", [(16, 129, 16, 72), (16, 256, 16, 80), (32, 161, 8, 70), (16, 193, 16, 67),
+                                          (16, 192, 16, 64), (16, 130, 16, 33), (16, 225, 16, 96), (32, 160, 8, 20),
+                                          (1, 64, 3, 66), (1, 127, 2, 79), (1, 97, 2, 31)])
+def test_encoder_attention_wide_workgroups(orc, dev, ns, tps, hc, hd):
+    """256 heads of sequences of 129 to 256 tokens run in workgroups of eight waves and two
+    tile buffers (the last three stay on four): partial last tiles of 1, 2, 32 and 33
+    keys, a whole last tile, query waves past the sequence's end, head dims whose last
+    dims run as 16 x 16 products (65 to 80) and dims that are no multiple of 4.  Bound:
+    TOL, as above."""
+    rng = np.random.default_rng(ns * 1000 + tps + hd)
+    q, k, v = (rng.standard_normal((ns * tps, hc * hd)).astype(np.float32) for _ in range(3))
+    shape = dict(n_seq=ns, tokens=tps, heads=hc, head_dim=hd)
+    got = _run(dev, q, k, v, **shape)
+    ref = orc.encoder_self_attention(q, k, v, n_threads=orc.env_threads(), **shape)
+    assert _within(got, ref), f"max abs {np.abs(got - ref).max():.3e}"
+
+
 def test_encoder_attention_sizes(dev):
     """A zero size is a no-op (the reference returns Ok for required == 0); negative sizes
     and head_dim > 256 are errors with a message."""
