@@ -22,12 +22,14 @@
 //    deltanet_chunk_prep_kernel (chunk, head): T, P and per-row scales; the
 //    Gram products on v_mfma_f32_16x16x4_f32, T by forward substitution in the
 //    diagonal 16x16 blocks and products below them.
-//    deltanet_chunk_scan_kernel (head, 16 state columns): the sequential chunk
-//    steps with the raw q / k rows as operands and their row scales applied to
-//    the products' rows; T X and P Delta on v_mfma_f32_16x16x4_f32, and K S0,
-//    Q S0 and the state update too for f32 / f16 rows, while bf16 rows (exact
-//    bf16 operands) run those three on v_mfma_f32_16x16x32_bf16 against the f32
-//    state / Delta cut into three exact bf16 pieces.
+//    deltanet_chunk_scan_kernel (head, 16 state columns; f32 / f16 rows): the
+//    sequential chunk steps with the raw q / k rows as operands and their row
+//    scales applied to the products' rows, all on v_mfma_f32_16x16x4_f32.
+//    deltanet_chunk_scan_bf16_kernel (the same blocks; bf16 rows, exact bf16
+//    operands): K S0, Q S0 and the state update on v_mfma_f32_16x16x32_bf16
+//    against the f32 state / Delta cut into three exact bf16 pieces, T X and P Delta
+//    on the f32 MFMA; four waves carry the chain from state to state, four beside
+//    them form the outputs.
 //    Non-finite values: the prep flags a chunk whose inputs, T or P are not all
 //    finite, the scan one whose X, Delta, O or new state are not.  The scan stops
 //    before such a chunk, keeping the state it started from, and the step kernel
