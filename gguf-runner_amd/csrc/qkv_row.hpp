@@ -1,6 +1,7 @@
-// One head row of the per-token Q/K/V preparation (qkv_prep.hip), shared with the
-// Turbo cache's fused token kernel (turbo_decode.hip) so that both compute the same
-// f32 rows: bias, QK RMSNorm, RoPE, Gemma q scale.
+// One head row of the per-token Q/K/V preparation for the Turbo cache's fused token
+// kernel (turbo_decode.hip): bias, QK RMSNorm, RoPE, Gemma q scale, the same f32 rows as
+// qkv_prep.hip, which has this body in place (there the function costs it a wave of
+// occupancy) and shares the loads and the RoPE table.
 #pragma once
 
 #include "gr_common.hpp"
