@@ -365,3 +365,36 @@ def test_large_f16_chunk_runs_in_overlapped_pieces(dev, orc, kv_dtype, window):
         start = max(0, t + 1 - window) if window else 0
         ref = orc.attention_token(q[t], kd, vd, fmt, n_heads, n_kv, d, start, t + 1)
         assert (np.abs(got[t] - ref) <= ATOL_16 + RTOL_16 * np.abs(ref)).all(), (t, float(np.abs(got[t] - ref).max()))
+
+
+@pytest.mark.parametrize("kv_dtype,block,m,n_heads,n_kv,d", [
+    ("Q8", False, 61, 32, 8, 128), ("Q8", True, 64, 32, 8, 128), ("F16", False, 55, 32, 8, 128),
+    ("BF16", False, 101, 16, 8, 128), ("F32", False, 131, 32, 4, 64), ("TURBO", False, 71, 32, 4, 128),
+    ("F16", False, 41, 16, 8, 256)])
+def test_prefill_chunk_fed_in_pieces_equals_small_chunks(dev, kv_dtype, block, m, n_heads, n_kv, d):
+    """A chunk of 1.25 MB or more of host rows is copied in pieces, each prepared while
+    the next is copied; the same rows as chunks of a few tokens (under the limit) leave
+    the same cache rows bit for bit, and outputs to the 16-bit bar."""
+    from gguf_runner_amd import ffi, runtime as rt
+    rng = np.random.default_rng(m + d)
+    p = rt.Config(n_layers=1, n_heads=n_heads, n_kv_heads=n_kv, head_dim=d, seq_len=m,
+                  kv_dtype=getattr(ffi, "DTYPE_" + kv_dtype), rope_mode=ffi.ROPE_NEOX, q8_block_scales=block,
+                  q_norm=1 + 0.1 * rng.standard_normal((1, d)).astype(np.float32),
+                  k_norm=1 + 0.1 * rng.standard_normal((1, d)).astype(np.float32))
+    whole, parts = rt.malloc_run_state(p), rt.malloc_run_state(p)
+    q, k, v = (rng.standard_normal((m, w)).astype(np.float32) for w in (p.q_dim, p.kv_dim, p.kv_dim))
+    assert 4 * (q.size + k.size + v.size) >= 5 << 18
+    a = rt.prefill_attention_chunk(p, whole, 0, 0, q, k, v)
+    b = np.concatenate([rt.prefill_attention_chunk(p, parts, 0, i, q[i:i + 8], k[i:i + 8], v[i:i + 8])
+                        for i in range(0, m, 8)])
+    assert (np.abs(a - b) <= ATOL_16 + RTOL_16 * np.abs(b)).all(), float(np.abs(a - b).max())
+    if kv_dtype == "TURBO":
+        x, y = rt.read_turbo_rows(p, whole, 0, 0, m), rt.read_turbo_rows(p, parts, 0, 0, m)
+        for name in x:
+            assert np.array_equal(x[name], y[name]), name
+        return
+    for x, y in zip(rt.read_kv_rows(p, whole, 0, 0, m), rt.read_kv_rows(p, parts, 0, 0, m)):
+        assert np.array_equal(x, y)
+    if kv_dtype == "Q8":
+        for x, y in zip(rt.read_kv_scales(p, whole, 0, 0, m), rt.read_kv_scales(p, parts, 0, 0, m)):
+            assert np.array_equal(x, y)

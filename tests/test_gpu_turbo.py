@@ -401,3 +401,47 @@ def test_turbo_large_chunk_runs_in_overlapped_pieces(orc, dev):
         ref = orc.attention_token_turbo(q[t], c, table, layer, n_heads, 0, t + 1)
         worst = max(worst, float(np.abs(got[t] - ref).max()))
     assert worst <= TOL, worst
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_turbo_combine_many_partials(orc, dev, d):
+    """Calls of up to 16 and 32 partials per head merge them with a workgroup per head:
+    heads with the full count, with one partial and with none, in one call."""
+    for top in (2048, 4097):
+        got, ref = _decode_case(orc, dev, n_heads=4, n_kv=2, d=d, starts=[0, 3, 5, 700],
+                                ends=[top, 10, 5, 1800], seq_len=top, seed=77 + d)
+        assert float(np.abs(got - ref).max()) <= TOL, (top, float(np.abs(got - ref).max()))
+        assert not got[2].any()
+
+
+@pytest.mark.parametrize("d,n_heads,n_kv,rope,rope_dim,norm", [
+    (128, 32, 8, "ROPE_NEOX", 0, True), (128, 40, 4, "ROPE_NEOX", 48, False),
+    (64, 32, 8, "ROPE_ADJACENT", 0, False), (64, 14, 2, "ROPE_NEOX", 0, True),
+    (256, 16, 4, "ROPE_NEOX", 64, True), (256, 8, 4, "ROPE_NONE", 0, True)])
+def test_turbo_token_kernel_equals_passes(dev, d, n_heads, n_kv, rope, rope_dim, norm):
+    """The same decode steps as one batch of more than 3072 head rows (preparation,
+    quantising write and query rotation as passes of their own) and as batches below it
+    (one launch): cache rows bit for bit the same, outputs to the fp32 bar."""
+    from gguf_runner_amd import ffi, runtime as rt
+    rows = n_heads + 2 * n_kv
+    n = 3072 // rows + 1
+    rng = np.random.default_rng(d + n_heads)
+    extra = {}
+    if norm:
+        extra = dict(q_norm=1 + 0.2 * rng.standard_normal((1, d)).astype(np.float32),
+                     k_norm=1 + 0.2 * rng.standard_normal((1, d)).astype(np.float32))
+    p = rt.Config(n_layers=1, n_heads=n_heads, n_kv_heads=n_kv, head_dim=d, seq_len=8, n_seq=n,
+                  kv_dtype=ffi.DTYPE_TURBO, rope_mode=getattr(ffi, rope), rope_dim=rope_dim, **extra)
+    whole, parts = rt.malloc_run_state(p), rt.malloc_run_state(p)
+    for pos in range(3):
+        q, k, v = (rng.standard_normal((n, w)).astype(np.float32) for w in (p.q_dim, p.kv_dim, p.kv_dim))
+        at = [pos] * n
+        a = rt.decode_layer_batch(p, whole, 0, list(range(n)), at, q, k, v)
+        cuts = [0, 1, n // 2, n]  # 1, about 1500 and about 1500 head rows
+        b = np.concatenate([rt.decode_layer_batch(p, parts, 0, list(range(i, j)), at[i:j], q[i:j], k[i:j], v[i:j])
+                            for i, j in zip(cuts, cuts[1:])])
+        assert float(np.abs(a - b).max()) <= TOL, (pos, float(np.abs(a - b).max()))
+    for sq in (0, 1, n // 2, n - 1):
+        x, y = rt.read_turbo_rows(p, whole, 0, 0, 3, seq=sq), rt.read_turbo_rows(p, parts, 0, 0, 3, seq=sq)
+        for name in x:
+            assert np.array_equal(x[name], y[name]), (sq, name)
