@@ -987,11 +987,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t bf_rsrc(const char* base, int 
                        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) << 32;
     return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)u, 0, __builtin_amdgcn_readfirstlane(bytes), 0x00020000);
 }
-__device__ __forceinline__ uint4 bf_load16(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
+// The bounds check covers the lane offset, not the scalar one, which stays 0 everywhere
+// here: what a load may read is its descriptor's range, and past it zero.
+__device__ __forceinline__ uint4 bf_load16(__amdgpu_buffer_rsrc_t r, int voff) {
+    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
 }
-__device__ __forceinline__ float4 bf_load4f(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
-    return __builtin_bit_cast(float4, bf_load16(r, voff, soff));
+__device__ __forceinline__ float4 bf_load4f(__amdgpu_buffer_rsrc_t r, int voff) {
+    return __builtin_bit_cast(float4, bf_load16(r, voff));
 }
 __device__ __forceinline__ dn_f32x4 bf_mma(const uint4& a, const uint4& b, dn_f32x4 c) {
     return mfma32<GR_DTYPE_BF16>(a, b, c);
@@ -1033,9 +1035,9 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
     // The loads run one chunk ahead: `roff` is the byte offset of the next chunk's rows
     // in q / k / v, `rbytes` the bytes of its rows (rows past the end of the sequence,
     // and every row past the last chunk, read as zero: they are past the descriptor),
-    // `blk` / `bbytes` its block.
+    // `blk` its block (past the last chunk: descriptors of no bytes).
     size_t roff = (size_t)h * D * 2;
-    int left = p.n_tokens, rbytes = 0, bbytes = kBfBytes;
+    int left = p.n_tokens, rbytes = 0;
     const char* blk = (const char*)p.ws + dn_ws_head(H) + (size_t)h * kBfBytes;
     auto bytes_of = [&]() { return left > 0 ? (min(C, left) - 1) * row + D * 2 : 0; };
     rbytes = bytes_of();
@@ -1044,12 +1046,15 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
         blk += (size_t)H * kBfBytes;
         left -= C;
         rbytes = bytes_of();
-        bbytes = left > 0 ? kBfBytes : 0;
     };
     auto rows_of = [&](const void* src) { return bf_rsrc((const char*)src + roff, rbytes); };
-    auto block_of = [&]() { return bf_rsrc(blk, bbytes); };
+    // `bytes` bytes of the block from `off` on
+    auto block_of = [&](int off, int bytes) { return bf_rsrc(blk + off, left > 0 ? bytes : 0); };
+    auto scales_of = [&]() { return block_of(kBfScale, kBfGl - kBfScale); };
     // gamma_last, flag
-    auto load_gl = [&]() { return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(block_of(), 0, kBfGl, 0)); };
+    auto load_gl = [&]() {
+        return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(block_of(kBfGl, 8), 0, 0, 0));
+    };
 
     if (tid == 0) flag = 0;
     int done = n_chunks;  // chunks completed
@@ -1082,14 +1087,14 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
         auto load_q = [&]() {
             const auto r = rows_of(p.q);
 #pragma unroll
-            for (int q = 0; q < 4; q++) qa[q] = bf_load16(r, qoff[q], 0);
+            for (int q = 0; q < 4; q++) qa[q] = bf_load16(r, qoff[q]);
         };
         auto load_p = [&]() {
-            const auto r = block_of();
+            // the wave's row of tiles; past the diagonal: past its end, zero
+            const auto r = block_of(kBfP + tp_tri(wave, 0) * 1024, (wave + 1) * 1024);
 #pragma unroll
-            for (int q = 0; q < 4; q++)  // past the diagonal: past the block, zero
-                pa[q] = bf_load4f(r, apos, q <= wave ? kBfP + tp_tri(wave, q) * 1024 : kBfBytes);
-            sq = bf_load4f(r, 4 * (16 * wave + 4 * g), kBfScale + 8 * C);
+            for (int q = 0; q < 4; q++) pa[q] = bf_load4f(r, apos + 1024 * q);
+            sq = bf_load4f(scales_of(), 4 * (16 * wave + 4 * g) + 8 * C);
         };
         // O of chunk n and its store, from Q S0 (aq) and the chunk's Delta
         dn_f32x4 aq[2];
@@ -1165,8 +1170,9 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
     for (int mt = 0; mt < 4; mt++) koff[mt] = bf_tok(mt, l16) * row + (32 * wave + 8 * g) * 2;
 #pragma unroll
     for (int i = 0; i < 4; i++) voff[i] = (tok0 + i) * row + (c0 + l16) * 2;
-    // T operands of k-steps 0 and 1 (w < 2 has no k-step 1: past the block, zero)
-    const int toff[2] = {kBfT + 3072 * (wave < 2 ? wave : 2 * wave - 2), wave < 2 ? kBfBytes : kBfT + 3072 * (2 * wave - 1)};
+    // T operands of k-steps 0 and 1, one after the other (w < 2 has no k-step 1: past the
+    // end, zero)
+    const int top = kBfT + 3072 * (wave < 2 ? wave : 2 * wave - 2), tbytes = wave < 2 ? 3072 : 6144;
     char* kl = Kl[wave];
     uint4 ka[4], ta[2][3];
     float4 sb, sx, sk;
@@ -1175,23 +1181,23 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
     auto load_k = [&]() {
         const auto r = rows_of(p.k);
 #pragma unroll
-        for (int mt = 0; mt < 4; mt++) ka[mt] = bf_load16(r, koff[mt], 0);
+        for (int mt = 0; mt < 4; mt++) ka[mt] = bf_load16(r, koff[mt]);
     };
     auto load_x = [&]() {
-        const auto r = block_of();
-        sb = bf_load4f(r, 4 * tok0, kBfScale);
-        sx = bf_load4f(r, 4 * tok0, kBfScale + 4 * C);
+        const auto r = scales_of();
+        sb = bf_load4f(r, 4 * tok0);
+        sx = bf_load4f(r, 4 * tok0 + 4 * C);
         const auto v = rows_of(p.v);
 #pragma unroll
         for (int i = 0; i < 4; i++) vr[i] = __builtin_amdgcn_raw_buffer_load_b16(v, voff[i], 0, 0);
     };
     auto load_t = [&]() {
-        const auto r = block_of();
+        const auto r = block_of(top, tbytes);
 #pragma unroll
         for (int ks = 0; ks < 2; ks++)
 #pragma unroll
-            for (int pc = 0; pc < 3; pc++) ta[ks][pc] = bf_load16(r, 16 * lane, toff[ks] + 1024 * pc);
-        sk = bf_load4f(r, 4 * tok0, kBfScale + 12 * C);
+            for (int pc = 0; pc < 3; pc++) ta[ks][pc] = bf_load16(r, 16 * lane + 3072 * ks + 1024 * pc);
+        sk = bf_load4f(scales_of(), 4 * tok0 + 12 * C);
     };
     // four values of the lane as slots 4 (w % 2) .. + 3 of lane (g, l % 16) of k-step w / 2
     auto put = [&](uint4 (*dst)[3][64], const float* x) {
