@@ -178,15 +178,14 @@ static_assert(kTpGl + 8 <= kTpBytes, "block layout");
 // which the scan loads straight into registers.  Wave w of the scan owns tokens
 // tok(w, m) = 32 (w / 2) + 8 (m / 4) + 4 (w % 2) + m % 4, m < 16, so that the four
 // results of a lane group g are half of the eight consecutive reduction slots
-// 8 g .. 8 g + 7 of a k-step of 32 tokens.  Six (w, k-step) operands (w < 2: k-step
-// 0; w >= 2: 0 and 1) as three exact bf16 pieces each (hi, mid, lo by truncation),
-// [operand][piece][lane]: row tok(w, l % 16), columns 32 ks + 8 (l / 16) ..; then P
-// and the rest as above.
+// 8 g .. 8 g + 7 of a k-step of 32 tokens.  Twelve operands (w, 16 columns q) (w < 2: q
+// = 0, 1; w >= 2: 0 .. 3), wave after wave: lane l holds row tok(w, l % 16), columns
+// 16 q + 4 (l / 16) ..; then P and the rest as above.
 constexpr int kBfT = 0;
-constexpr int kBfP = kBfT + 18 * 1024;
+constexpr int kBfP = kBfT + 12 * 1024;
 constexpr int kBfScale = kBfP + kTpTiles * 1024;
 constexpr int kBfGl = kBfScale + 4 * kChunk * 4;
-constexpr int kBfBytes = 30 * 1024;
+constexpr int kBfBytes = kBfGl + 256;
 static_assert(kBfGl + 8 <= kBfBytes, "block layout");
 __device__ __forceinline__ int bf_tok(int w, int m) { return 32 * (w >> 1) + 8 * (m >> 2) + 4 * (w & 1) + (m & 3); }
 
@@ -529,20 +528,12 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
     }
     if constexpr (BF) {
         __syncthreads();
-        // T as operand pieces: wave w takes operands w and w + 4
+        // T as operands: wave w takes operands w, w + 4 and w + 8
 #pragma unroll
-        for (int u = 0; u < 2; u++) {
+        for (int u = 0; u < 3; u++) {
             const int op = wave + 4 * u;
-            if (op >= 6) break;
-            const int w = op < 2 ? op : (op + 2) >> 1, ks = op < 2 ? 0 : op & 1;
-            const float* src = tm + bf_tok(w, l16) * AMS + 32 * ks + 8 * g;
-            uint2 lo[3], hi[3];
-            dn_split3x4(src, lo);
-            dn_split3x4(src + 4, hi);
-#pragma unroll
-            for (int pc = 0; pc < 3; pc++)
-                *(uint4*)(blk + kBfT + ((3 * op + pc) * 64 + lane) * 16) =
-                    make_uint4(lo[pc].x, lo[pc].y, hi[pc].x, hi[pc].y);
+            const int w = op < 4 ? op >> 1 : 1 + (op >> 2), q = op < 4 ? op & 1 : op & 3;
+            *(float4*)(blk + kBfT + (op * 64 + lane) * 16) = *(const float4*)(tm + bf_tok(w, l16) * AMS + 16 * q + 4 * g);
         }
     }
     if (nf != 0.0f) bad = 1;
@@ -964,16 +955,15 @@ __global__ __launch_bounds__(kChunkThreads, 1) void deltanet_chunk_scan_kernel(c
 // the next chunk.  Products over the 128 state rows are then sums over the waves.  Per
 // chunk the chain waves compute
 //   1. K S0 over the wave's 32 rows, all 64 tokens                -> LDS (partial sums)
-//   2. X = beta V - (beta gamma / |k|) sum_w (K S0)_w, 16 tokens   -> LDS (pieces)
+//   2. X = beta V - (beta gamma / |k|) sum_w (K S0)_w, 16 tokens   -> LDS (f32)
 //   3. Delta = T X, 16 tokens, plain                               -> LDS (f32)
 //      and scaled by (gamma_last / gamma) / |k|                    -> LDS (pieces)
 //   4. S' = gamma_last S0 + K^T (scaled Delta), 32 rows            -> LDS (pieces)
 // with a barrier after each of 1 - 3, and the output waves 4 .. 7 follow beside them,
 // 16 tokens each: Q S0 beside step 3, O = (gamma / |q| sqrt(d)) Q S0 + P Delta beside
-// step 4.  f32 x f32 products take the six piece products down to 2^-16 (hi
-// hi, hi mid, mid hi, hi lo, mid mid, lo hi), bf16 x f32 ones all three (a bf16 MFMA
-// has 8 times the reduction length of an f32 one at half its time); P Delta stays on
-// the f32 MFMA.  Global operands go straight into registers, each loaded for the next
+// step 4.  bf16 x f32 products take all three pieces (a bf16 MFMA has 8 times the
+// reduction length of an f32 one at half its time); T X and P Delta, f32 x f32, are on the
+// f32 MFMA.  Global operands go straight into registers, each loaded for the next
 // chunk right after its last use in this one; K^T comes from the wave's own K
 // fragments through LDS.  What bounds it: the dependent steps of one chunk (LDS
 // round trips, barriers, the VALU work of cutting values into pieces) and the output
@@ -998,23 +988,14 @@ __device__ __forceinline__ float4 bf_load4f(__amdgpu_buffer_rsrc_t r, int voff) 
 __device__ __forceinline__ dn_f32x4 bf_mma(const uint4& a, const uint4& b, dn_f32x4 c) {
     return mfma32<GR_DTYPE_BF16>(a, b, c);
 }
-// six piece products of A (a[0..2]) and B (b[0..2]): three chains
-__device__ __forceinline__ void bf_mma6(const uint4* a, const uint4* b, dn_f32x4* acc) {
-    acc[0] = bf_mma(a[0], b[0], acc[0]);
-    acc[1] = bf_mma(a[0], b[1], acc[1]);
-    acc[2] = bf_mma(a[1], b[0], acc[2]);
-    acc[1] = bf_mma(a[0], b[2], acc[1]);
-    acc[2] = bf_mma(a[1], b[1], acc[2]);
-    acc[1] = bf_mma(a[2], b[0], acc[1]);
-}
 
 constexpr int kBfThreads = 512;
 
 __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel(const DeltaNetLaunch p) {
     constexpr int C = kChunk, D = 128, NC = kScanCols;
     __shared__ __attribute__((aligned(16))) float4 Pk[4][4][64];  // [token tile][wave][lane]
-    __shared__ __attribute__((aligned(16))) uint4 Xp[2][3][64];   // [k-step][piece][lane]
-    __shared__ __attribute__((aligned(16))) uint4 Ds[2][3][64];   // scaled Delta
+    __shared__ __attribute__((aligned(16))) float4 Xl[4][64];     // X [wave][lane]
+    __shared__ __attribute__((aligned(16))) uint4 Ds[2][3][64];   // scaled Delta [k-step][piece][lane]
     __shared__ __attribute__((aligned(16))) float4 Dl[4][64];     // Delta [wave][lane]
     __shared__ __attribute__((aligned(16))) uint4 Sp[4][3][64];   // state [k-step][piece][lane]
     // K of a chain wave's 32 dims: token t's 16-byte chunk c at c ^ (t / 8 % 4)
@@ -1056,6 +1037,11 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
         return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(block_of(kBfGl, 8), 0, 0, 0));
     };
 
+    // values of tokens 16 q + 4 g + i in the chain waves' layout: wave 2 (q / 2) + g % 2
+    auto rows16 = [&](const float4 (*x)[64], int q) {
+        return x[2 * (q >> 1) + (g & 1)][16 * (2 * (q & 1) + (g >> 1)) + l16];
+    };
+
     if (tid == 0) flag = 0;
     int done = n_chunks;  // chunks completed
     int c = 0;
@@ -1071,13 +1057,9 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
 
     if (wave8 >= 4) {
         // output waves: tokens 16 w + m
-        int qoff[4], dlane[4];
+        int qoff[4];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            qoff[q] = (16 * wave + l16) * row + (32 * q + 8 * g) * 2;
-            // Delta of tokens 16 q + 4 g + i: chain wave 2 (q / 2) + g % 2
-            dlane[q] = (2 * (q >> 1) + (g & 1)) * 64 + 16 * (2 * (q & 1) + (g >> 1)) + l16;
-        }
+        for (int q = 0; q < 4; q++) qoff[q] = (16 * wave + l16) * row + (32 * q + 8 * g) * 2;
         const int orow = H * D * 4;
         const int ooff = (16 * wave + 4 * g) * orow + (c0 + l16) * 4;
         uint4 qa[4];
@@ -1104,7 +1086,7 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
             dn_f32x4 o0 = zero, o1 = zero;
             float4 b[4];
 #pragma unroll
-            for (int q = 0; q < 4; q++) b[q] = ((const float4*)Dl)[dlane[q]];
+            for (int q = 0; q < 4; q++) b[q] = rows16(Dl, q);
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 o0 = mfma4(pa[q].x, b[q].x, o0);
@@ -1170,12 +1152,11 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
     for (int mt = 0; mt < 4; mt++) koff[mt] = bf_tok(mt, l16) * row + (32 * wave + 8 * g) * 2;
 #pragma unroll
     for (int i = 0; i < 4; i++) voff[i] = (tok0 + i) * row + (c0 + l16) * 2;
-    // T operands of k-steps 0 and 1, one after the other (w < 2 has no k-step 1: past the
-    // end, zero)
-    const int top = kBfT + 3072 * (wave < 2 ? wave : 2 * wave - 2), tbytes = wave < 2 ? 3072 : 6144;
+    // the wave's T operands (w < 2 has two: past the end, zero)
+    const int top = kBfT + 1024 * (wave < 2 ? 2 * wave : 4 * wave - 4), tbytes = wave < 2 ? 2048 : 4096;
     char* kl = Kl[wave];
-    uint4 ka[4], ta[2][3];
-    float4 sb, sx, sk;
+    uint4 ka[4];
+    float4 ta[4], sb, sx, sk;
     uint32_t vr[4];
     uint2 gb;
     auto load_k = [&]() {
@@ -1194,17 +1175,8 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
     auto load_t = [&]() {
         const auto r = block_of(top, tbytes);
 #pragma unroll
-        for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-            for (int pc = 0; pc < 3; pc++) ta[ks][pc] = bf_load16(r, 16 * lane + 3072 * ks + 1024 * pc);
+        for (int q = 0; q < 4; q++) ta[q] = bf_load4f(r, 16 * lane + 1024 * q);
         sk = bf_load4f(scales_of(), 4 * tok0 + 12 * C);
-    };
-    // four values of the lane as slots 4 (w % 2) .. + 3 of lane (g, l % 16) of k-step w / 2
-    auto put = [&](uint4 (*dst)[3][64], const float* x) {
-        uint2 pcs[3];
-        dn_split3x4(x, pcs);
-#pragma unroll
-        for (int pc = 0; pc < 3; pc++) *((uint2*)&dst[wave >> 1][pc][lane] + (wave & 1)) = pcs[pc];
     };
     // the wave's state rows 32 w + 8 g + 4 tt + i of column c0 + l16
     dn_f32x4 st[2], s0own[2];
@@ -1273,22 +1245,25 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
                 asm volatile("" : "+v"(vr[i]));
                 xv[i] = b4[i] * __uint_as_float(vr[i] << 16) - x4[i] * ks[i];
             }
-            put(Xp, xv);
+            Xl[wave][lane] = make_float4(xv[0], xv[1], xv[2], xv[3]);
         }
         load_x();
         dn_lds_barrier();  // 2
         // 3.
         uint4 kt[2][2];
         {
-            dn_f32x4 acc[3] = {zero, zero, zero};
-            uint4 xb[2][3];
+            dn_f32x4 d0 = zero, d1 = zero;
+            float4 xb[4];
 #pragma unroll
-            for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-                for (int pc = 0; pc < 3; pc++) xb[ks][pc] = Xp[ks][pc][lane];
+            for (int q = 0; q < 4; q++) xb[q] = rows16(Xl, q);
             __builtin_amdgcn_sched_barrier(0);  // every read issued before the first product
-            bf_mma6(ta[0], xb[0], acc);
-            bf_mma6(ta[1], xb[1], acc);
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                d0 = mfma4(ta[q].x, xb[q].x, d0);
+                d1 = mfma4(ta[q].y, xb[q].y, d1);
+                d0 = mfma4(ta[q].z, xb[q].z, d0);
+                d1 = mfma4(ta[q].w, xb[q].w, d1);
+            }
             // K^T (rows 8 m / 4 + 4 tt + m % 4 of the wave's dims, tokens 32 ks + 8 g ..): lane i
             // of a 16-lane group supplies token k0 + i / 4, half tt of chunk i % 4, and
             // receives dim i of the four chunks' halves
@@ -1306,14 +1281,12 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
                     }
                     kt[tt][ks] = make_uint4(part[0].x, part[0].y, part[1].x, part[1].y);
                 }
-            const dn_f32x4 dl = acc[0] + (acc[1] + acc[2]);
-            const float k4[4] = {sk.x, sk.y, sk.z, sk.w};
-            float ds[4];
+            const dn_f32x4 dl = d0 + d1;
+            const float ds[4] = {dl[0] * sk.x, dl[1] * sk.y, dl[2] * sk.z, dl[3] * sk.w};
+            uint2 pcs[3];  // slots 4 (w % 2) .. + 3 of lane (g, l % 16) of k-step w / 2
+            dn_split3x4(ds, pcs);
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                ds[i] = dl[i] * k4[i];
-            }
-            put(Ds, ds);
+            for (int pc = 0; pc < 3; pc++) *((uint2*)&Ds[wave >> 1][pc][lane] + (wave & 1)) = pcs[pc];
             Dl[wave][lane] = make_float4(dl[0], dl[1], dl[2], dl[3]);
         }
         load_t();

@@ -200,6 +200,30 @@ def test_deltanet_bf16_scan_nonfinite(orc, dev):
     assert not bad.transpose(0, 2, 1)[cols].any()
 
 
+def test_deltanet_bf16_scan_product_rounding(dev):
+    """T X of the bf16 scan, a product of two f32 operands, one term at a time: k_0 = e_0, k_1 =
+    e_0 + e_1, no decay, a zero state and v_1 = 0 leave T[1][0] = -beta_1, X[0] = beta_0 v_0 and
+    row 1 of the state = -beta_1 beta_0 v_0, with every other step exact (v_0 powers of
+    two).  Bound: twice the f32 rounding of the product.  Half the heads have a leading
+    one, zeros and then ones, values of which the six largest products of truncated bf16
+    pieces leave out 2^-21."""
+    from gguf_runner_amd import ops
+    H, d = 64, 128
+    rng = np.random.default_rng(8)
+    beta = rng.uniform(0.5, 1.0, (2, H)).astype(np.float32)
+    beta[:, ::2] = 0.5 + (0xffff - rng.integers(0, 9, (2, H // 2))) * np.float32(2.0 ** -24)
+    q, k, v = (np.zeros((2, H, d), np.float32) for _ in range(3))
+    k[:, :, 0] = k[1, :, 1] = 1
+    v[0] = 2.0 ** (np.arange(d) % 16 - 8)
+    st = torch.zeros((H, d, d), device=dev)
+    ops.DeltaNetCall(*(torch.from_numpy(x).to(dev).bfloat16() for x in (q, k, v)), torch.zeros((2, H), device=dev),
+                     torch.from_numpy(beta).to(dev), st, torch.empty((2, H, d), device=dev), l2norm=False, algo=2)()
+    S = st.cpu().numpy().astype(np.float64)
+    want = -(beta[0].astype(np.float64) * beta[1])[:, None] * v[0]
+    rel = np.abs(S[:, 1] / want - 1).max()
+    assert rel <= 2.0 ** -23, np.log2(rel)
+
+
 @pytest.mark.parametrize("d,algo,fmt_name", [(64, 1, "F32"), (64, 0, "BF16"), (256, 1, "F32"), (256, 2, "F16")])
 def test_deltanet_state_sizes_64_and_256(orc, dev, d, algo, fmt_name):
     """State sizes other than 128 (the reference takes any ssm_state_size, math.rs:566):
