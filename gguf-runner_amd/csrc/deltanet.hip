@@ -178,15 +178,23 @@ static_assert(kTpGl + 8 <= kTpBytes, "block layout");
 // which the scan loads straight into registers.  Wave w of the scan owns tokens
 // tok(w, m) = 32 (w / 2) + 8 (m / 4) + 4 (w % 2) + m % 4, m < 16, so that the four
 // results of a lane group g are half of the eight consecutive reduction slots
-// 8 g .. 8 g + 7 of a k-step of 32 tokens.  Twelve operands (w, 16 columns q) (w < 2: q
-// = 0, 1; w >= 2: 0 .. 3), wave after wave: lane l holds row tok(w, l % 16), columns
-// 16 q + 4 (l / 16) ..; then P and the rest as above.
-constexpr int kBfT = 0;
-constexpr int kBfP = kBfT + 12 * 1024;
-constexpr int kBfScale = kBfP + kTpTiles * 1024;
-constexpr int kBfGl = kBfScale + 4 * kChunk * 4;
-constexpr int kBfBytes = kBfGl + 256;
-static_assert(kBfGl + 8 <= kBfBytes, "block layout");
+// 8 g .. 8 g + 7 of a k-step of 32 tokens.  Operand (w, q) of 16 columns (w < 2: q = 0, 1;
+// w >= 2: 0 .. 3), wave after wave: lane l holds row tok(w, l % 16), columns
+// 16 q + 4 (l / 16) ..; of a wave's last operand only lanes of m = l % 16 >= 8 (the other rows
+// lie above these columns, zero), 512 bytes: as large as the ten tiles.  P and the rest as
+// above.
+__host__ __device__ constexpr int bf_t_ops(int w) { return w < 2 ? 2 : 4; }
+__host__ __device__ constexpr int bf_t_bytes(int w) { return bf_t_ops(w) * 1024 - 512; }
+__host__ __device__ constexpr int bf_t_base(int w) {
+    return kTpT + (w > 0 ? bf_t_bytes(0) : 0) + (w > 1 ? bf_t_bytes(1) : 0) + (w > 2 ? bf_t_bytes(2) : 0);
+}
+static_assert(bf_t_base(3) + bf_t_bytes(3) == kTpP, "block layout");
+// byte of lane l of operand q within the wave's (none: past every descriptor, read as zero)
+constexpr int kBfNone = 0x40000000;
+__device__ __forceinline__ int bf_t_off(int w, int q, int l) {
+    if (q + 1 < bf_t_ops(w)) return 1024 * q + 16 * l;
+    return (l & 15) < 8 ? kBfNone : 1024 * q + 16 * (8 * (l >> 4) + (l & 7));
+}
 __device__ __forceinline__ int bf_tok(int w, int m) { return 32 * (w >> 1) + 8 * (m >> 2) + 4 * (w & 1) + (m & 3); }
 
 // Workspace: [H][kScanBlocks] i32 chunks completed by each scan block (256-byte
@@ -313,7 +321,7 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
     const int c = blockIdx.x, h = blockIdx.y, H = p.n_heads;
     const int t0 = c * C;
     const int Cn = min(C, p.n_tokens - t0);
-    char* blk = (char*)p.ws + dn_ws_head(H) + ((size_t)c * H + h) * (BF ? kBfBytes : kTpBytes);
+    char* blk = (char*)p.ws + dn_ws_head(H) + ((size_t)c * H + h) * kTpBytes;
     if (tid == 0) bad = 0;
     __syncthreads();
 
@@ -459,7 +467,7 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
                 const float pr = RAW ? qi[t] * ks * acc[u][i] : acc[u][i];
                 const float v = s <= t ? dec * pr : 0.0f;
                 nf = fmaf(v, 0.0f, nf);
-                *(float*)(blk + (BF ? kBfP : kTpP) + tt * 1024 + 4 * tp_elem(tl, l16)) = v;
+                *(float*)(blk + kTpP + tt * 1024 + 4 * tp_elem(tl, l16)) = v;
             }
         }
     }
@@ -522,25 +530,24 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
                 else *(float*)(blk + kTpT + tp_tri(i, wave) * 1024 + 4 * tp_elem(4 * g + e, l16)) = tb[n][e];
             }
         }
-        // the two blocks above the diagonal that T's operands read
-        if (BF && wave == 3)
-            for (int e = lane; e < 512; e += 64) tm[((e >> 8) * 32 + ((e >> 4) & 15)) * AMS + (e >> 8) * 32 + 16 + (e & 15)] = 0.0f;
     }
     if constexpr (BF) {
         __syncthreads();
-        // T as operands: wave w takes operands w, w + 4 and w + 8
+        // T as operands: the twelve shared out, three to a wave
 #pragma unroll
         for (int u = 0; u < 3; u++) {
             const int op = wave + 4 * u;
             const int w = op < 4 ? op >> 1 : 1 + (op >> 2), q = op < 4 ? op & 1 : op & 3;
-            *(float4*)(blk + kBfT + (op * 64 + lane) * 16) = *(const float4*)(tm + bf_tok(w, l16) * AMS + 16 * q + 4 * g);
+            const int off = bf_t_off(w, q, lane);
+            if (off != kBfNone)
+                *(float4*)(blk + bf_t_base(w) + off) = *(const float4*)(tm + bf_tok(w, l16) * AMS + 16 * q + 4 * g);
         }
     }
     if (nf != 0.0f) bad = 1;
     // 4. row scales, gamma_last, flag
     if (tid < C) {
         const int t = tid;
-        float* sc = (float*)(blk + (BF ? kBfScale : kTpScale));
+        float* sc = (float*)(blk + kTpScale);
         const float v0 = bt[t], v1 = bt[t] * gm[t] * ki[t], v2 = gm[t] * qi[t], v3 = kf[t] * ki[t];
         sc[t] = v0;
         sc[C + t] = v1;
@@ -550,11 +557,11 @@ __global__ __launch_bounds__(kChunkThreads, DT == GR_DTYPE_F32 ? 2 : 4) void del
         if (t == C - 1) {
             const float gl = gm[C - 1];
             if (!is_finite_f(gl)) bad = 1;
-            *(float*)(blk + (BF ? kBfGl : kTpGl)) = gl;
+            *(float*)(blk + kTpGl) = gl;
         }
     }
     __syncthreads();
-    if (tid == 0) *(int*)(blk + (BF ? kBfGl : kTpGl) + 4) = bad;
+    if (tid == 0) *(int*)(blk + kTpGl + 4) = bad;
 }
 
 // Raw buffer access: a buffer descriptor (base, stride 0, num_records = `bytes`:
@@ -1019,22 +1026,22 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
     // `blk` its block (past the last chunk: descriptors of no bytes).
     size_t roff = (size_t)h * D * 2;
     int left = p.n_tokens, rbytes = 0;
-    const char* blk = (const char*)p.ws + dn_ws_head(H) + (size_t)h * kBfBytes;
+    const char* blk = (const char*)p.ws + dn_ws_head(H) + (size_t)h * kTpBytes;
     auto bytes_of = [&]() { return left > 0 ? (min(C, left) - 1) * row + D * 2 : 0; };
     rbytes = bytes_of();
     auto next_chunk = [&]() {
         roff += (size_t)C * row;
-        blk += (size_t)H * kBfBytes;
+        blk += (size_t)H * kTpBytes;
         left -= C;
         rbytes = bytes_of();
     };
     auto rows_of = [&](const void* src) { return bf_rsrc((const char*)src + roff, rbytes); };
     // `bytes` bytes of the block from `off` on
     auto block_of = [&](int off, int bytes) { return bf_rsrc(blk + off, left > 0 ? bytes : 0); };
-    auto scales_of = [&]() { return block_of(kBfScale, kBfGl - kBfScale); };
+    auto scales_of = [&]() { return block_of(kTpScale, kTpGl - kTpScale); };
     // gamma_last, flag
     auto load_gl = [&]() {
-        return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(block_of(kBfGl, 8), 0, 0, 0));
+        return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(block_of(kTpGl, 8), 0, 0, 0));
     };
 
     // values of tokens 16 q + 4 g + i in the chain waves' layout: wave 2 (q / 2) + g % 2
@@ -1073,7 +1080,7 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
         };
         auto load_p = [&]() {
             // the wave's row of tiles; past the diagonal: past its end, zero
-            const auto r = block_of(kBfP + tp_tri(wave, 0) * 1024, (wave + 1) * 1024);
+            const auto r = block_of(kTpP + tp_tri(wave, 0) * 1024, (wave + 1) * 1024);
 #pragma unroll
             for (int q = 0; q < 4; q++) pa[q] = bf_load4f(r, apos + 1024 * q);
             sq = bf_load4f(scales_of(), 4 * (16 * wave + 4 * g) + 8 * C);
@@ -1152,8 +1159,11 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
     for (int mt = 0; mt < 4; mt++) koff[mt] = bf_tok(mt, l16) * row + (32 * wave + 8 * g) * 2;
 #pragma unroll
     for (int i = 0; i < 4; i++) voff[i] = (tok0 + i) * row + (c0 + l16) * 2;
-    // the wave's T operands (w < 2 has two: past the end, zero)
-    const int top = kBfT + 1024 * (wave < 2 ? 2 * wave : 4 * wave - 4), tbytes = wave < 2 ? 2048 : 4096;
+    // the wave's T operands (w < 2 has two: past them, zero)
+    const int top = bf_t_base(wave), tbytes = bf_t_bytes(wave);
+    int toff[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) toff[q] = q < bf_t_ops(wave) ? bf_t_off(wave, q, lane) : kBfNone;
     char* kl = Kl[wave];
     uint4 ka[4];
     float4 ta[4], sb, sx, sk;
@@ -1175,7 +1185,7 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
     auto load_t = [&]() {
         const auto r = block_of(top, tbytes);
 #pragma unroll
-        for (int q = 0; q < 4; q++) ta[q] = bf_load4f(r, 16 * lane + 1024 * q);
+        for (int q = 0; q < 4; q++) ta[q] = bf_load4f(r, toff[q]);
         sk = bf_load4f(scales_of(), 4 * tok0 + 12 * C);
     };
     // the wave's state rows 32 w + 8 g + 4 tt + i of column c0 + l16
@@ -1342,7 +1352,7 @@ __global__ __launch_bounds__(kBfThreads, 1) void deltanet_chunk_scan_bf16_kernel
 size_t deltanet_chunked_ws_bytes(int n_tokens, int n_heads, int head_dim, int chunk) {
     if (head_dim != 128 || chunk != kChunk || n_tokens <= 0 || n_heads <= 0) return 0;
     const size_t n_chunks = (size_t)(n_tokens + kChunk - 1) / kChunk;
-    return dn_ws_head(n_heads) + n_chunks * n_heads * kBfBytes;  // (the larger of the two blocks)
+    return dn_ws_head(n_heads) + n_chunks * n_heads * kTpBytes;
 }
 
 // The token recurrence at any supported state size (64, 128, 256: 32 value

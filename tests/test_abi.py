@@ -166,3 +166,17 @@ def test_prefill_rejects_misaligned_norm_weights(pkg):
     a.q_norm, a.k_norm = (1 << 20) + 8, 1 << 21
     assert L.gr_prefill_attention(ctypes.byref(a), None) == ffi.GR_ERR_ARG
     assert b"q_norm and k_norm must be 16-byte aligned" in L.gr_last_error()
+
+
+def test_deltanet_workspace_is_one_block_per_chunk_and_head(pkg):
+    """gr_deltanet_workspace_size: the completed-chunk counts (256-byte aligned), then 22 KB per
+    (chunk of 64, head), whatever the row type; nothing for the token recurrence."""
+    from gguf_runner_amd import ffi
+    L = ffi.lib()
+    for dtype in (ffi.DTYPE_F32, ffi.DTYPE_F16, ffi.DTYPE_BF16):
+        for T, H in ((1, 16), (64, 1), (65, 3), (4096, 16)):
+            a = ffi.DeltaNetArgs()
+            a.n_tokens, a.n_heads, a.head_dim, a.in_dtype, a.algo = T, H, 128, dtype, ffi.DELTANET_CHUNKED
+            assert L.gr_deltanet_workspace_size(ctypes.byref(a)) == -(-32 * H // 256) * 256 + -(-T // 64) * H * 22 * 1024
+            a.algo = ffi.DELTANET_RECURRENT
+            assert L.gr_deltanet_workspace_size(ctypes.byref(a)) == 0
