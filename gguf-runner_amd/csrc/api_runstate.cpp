@@ -101,6 +101,7 @@ struct MappedRows {
     int finish() {
         const hipError_t e = hipStreamSynchronize(s->stream);
         if (e != hipSuccess) return hip_fail(e, "stream synchronize");
+        s->mapped_used = std::max(s->mapped_used, off);
         for (const Out& o : outs) host_copy(o.dst, s->mapped + o.off, o.bytes);
         return GR_OK;
     }
@@ -925,12 +926,16 @@ static int prefill_rows(gr_run_state* s, int32_t seq, int32_t layer, int64_t bas
     const PrepFeed* fp = nullptr;
     if (mp) {
         // From 1.25 MB of input rows on they are copied in up to four pieces, each read by
-        // its own prep launch while the host copies the next: 64 tokens, 32 / 8 heads, Q8,
-        // 166 -> 153 us per call.  (1 MB, 16 / 8 heads: four pieces 2-5% slower, the launches
-        // cost what the overlap gives.)
+        // its own prep launch while the host copies the next.  64 tokens after 1984, 32 / 8
+        // heads, Q8, per call: 175 -> 155 us with rows that the host caches hold, 194 -> 163
+        // with rows that they do not; 100 tokens 214 -> 194 and 233 -> 210.  (1 MB, 16 / 8
+        // heads: four pieces 2-5% slower, the launches cost what the overlap gives.)  Not
+        // into memory of the buffer that no call has used yet: the host's first touch of its
+        // pages bounds that copy, which two copy threads share and one thread feeding does
+        // not (first call of a state with a new buffer 1000 us, fed 1100).
         const size_t bytes = qb + 2 * kb;
         const int n_feed = bytes < (size_t(5) << 18) ? 1 : (int)std::min<size_t>({4, bytes / (size_t(3) << 17), (size_t)m});
-        const bool fed = n_feed > 1;
+        const bool fed = n_feed > 1 && s->mapped_used >= bytes;
         qin[0] = fed ? mr.reserve<float>((size_t)m * s->q_dim) : mr.in(q, (size_t)m * s->q_dim);
         kin[0] = fed ? mr.reserve<float>((size_t)m * s->kv_dim) : mr.in(k, (size_t)m * s->kv_dim);
         vin[0] = fed ? mr.reserve<float>((size_t)m * s->kv_dim) : mr.in(v, (size_t)m * s->kv_dim);

@@ -58,6 +58,7 @@ struct gr_run_state {
     // DMA copy on either side (allocated on first use, kMappedBytes).
     char* mapped = nullptr;      // host address
     char* mapped_dev = nullptr;  // the same memory's device address
+    size_t mapped_used = 0;      // bytes from its start that a call has used
     bool mapped_failed = false;  // allocation refused once: the copy path is used
 };
 

@@ -373,8 +373,11 @@ def test_large_f16_chunk_runs_in_overlapped_pieces(dev, orc, kv_dtype, window):
     ("F16", False, 41, 16, 8, 256)])
 def test_prefill_chunk_fed_in_pieces_equals_small_chunks(dev, kv_dtype, block, m, n_heads, n_kv, d):
     """A chunk of 1.25 MB or more of host rows is copied in pieces, each prepared while
-    the next is copied; the same rows as chunks of a few tokens (under the limit) leave
-    the same cache rows bit for bit, and outputs to the 16-bit bar."""
+    the next is copied (from the state's second chunk on: the first finds a new buffer);
+    the same rows as chunks of a few tokens (under the limit) leave the same cache
+    rows bit for bit, and outputs to the 16-bit bar.  The first chunk has other rows, which
+    the second overwrites; then the second's rows once more on a state of their own,
+    unfed: the same outputs bit for bit."""
     from gguf_runner_amd import ffi, runtime as rt
     rng = np.random.default_rng(m + d)
     p = rt.Config(n_layers=1, n_heads=n_heads, n_kv_heads=n_kv, head_dim=d, seq_len=m,
@@ -384,7 +387,9 @@ def test_prefill_chunk_fed_in_pieces_equals_small_chunks(dev, kv_dtype, block, m
     whole, parts = rt.malloc_run_state(p), rt.malloc_run_state(p)
     q, k, v = (rng.standard_normal((m, w)).astype(np.float32) for w in (p.q_dim, p.kv_dim, p.kv_dim))
     assert 4 * (q.size + k.size + v.size) >= 5 << 18
+    rt.prefill_attention_chunk(p, whole, 0, 0, -q, 1 - k, 1 - v)
     a = rt.prefill_attention_chunk(p, whole, 0, 0, q, k, v)
+    assert np.array_equal(a, rt.prefill_attention_chunk(p, rt.malloc_run_state(p), 0, 0, q, k, v))
     b = np.concatenate([rt.prefill_attention_chunk(p, parts, 0, i, q[i:i + 8], k[i:i + 8], v[i:i + 8])
                         for i in range(0, m, 8)])
     assert (np.abs(a - b) <= ATOL_16 + RTOL_16 * np.abs(b)).all(), float(np.abs(a - b).max())
