@@ -927,9 +927,8 @@ static PfSplitShape pf_split_shape(int head_dim) {
 }
 
 // Split or not: in tiles of 128 rows x BN keys, the unsplit launch takes its longest
-// pair of blocks (it has at most one workgroup per CU here); the split one at least
-// one piece and its share of all tiles, 1.1 for the uneven finish, a tile for the
-// combine launch and 0.03 (d128) per workgroup for its partials.  Fitted to 74
+// pair of blocks (it has at most one workgroup per CU here); the split one as
+// pf_split_choose says, 0.03 (d128) per workgroup for its partials.  Fitted to 74
 // launches, 16 to 4096 tokens after 0 to 8000, five head shapes: the rule takes
 // the slower side by at most 4%.  MI355X, us per call (prep included), unsplit ->
 // split: 32 / 8 heads d128, 64 tokens after 4000 78.5 -> 29, 512 after 8000 302 -> 92,
@@ -942,16 +941,12 @@ PrefillSplit prefill_split_plan(int n_tokens, int n_heads, int n_kv_heads, int h
     if (n_tokens <= 0) return {};
     const int n_qb = (n_tokens - 1) / sh.bm + 1;
     if ((int64_t)n_heads * ((n_qb + 1) / 2) > kPfCUs) return {};
-    const PrefillSplit s = pf_split_plan(n_tokens, n_heads, n_kv_heads, base_pos, window, bidirectional, sh.bm, sh.bn,
-                                         sh.slots, 128 / sh.bn);
-    if (s.n_splits == 0) return s;
     auto block = [&](int qb) {
         return pf_split_tiles(qb, sh.bm, sh.bn, n_tokens, 1, base_pos, window, bidirectional);
     };
     const float whole = (float)(block(n_qb - 1) + (n_qb > 1 ? block(0) : 0));
-    const float share = (float)s.tiles / kPfCUs;
-    const float cost = 1.1f * (share > s.ct ? share : (float)s.ct) + 1.0f + 0.03f * s.wgs * head_dim / 128;
-    return cost < whole ? s : PrefillSplit{};
+    return pf_split_choose(n_tokens, n_heads, n_kv_heads, base_pos, window, bidirectional, sh.bm, sh.bn, sh.slots,
+                           128 / sh.bn, whole, kPfCUs, 0.03f * head_dim / 128);
 }
 
 size_t prefill_split_ws_bytes(int head_dim) {

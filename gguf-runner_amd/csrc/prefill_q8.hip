@@ -583,12 +583,9 @@ PrefillSplit q8_plan(int n_tokens, int n_heads, int n_kv_heads, int base_pos, in
     if (n_tokens <= 0) return {};
     const int n_qb = (n_tokens - 1) / BM + 1;
     if ((int64_t)n_heads * n_qb > kQ8CUs) return {};
-    const PrefillSplit s = pf_split_plan(n_tokens, n_heads, n_kv_heads, base_pos, window, bidirectional, BM, BN, kQ8CUs, 1);
-    if (s.n_splits == 0) return s;
     const float whole = (float)pf_split_tiles(n_qb - 1, BM, BN, n_tokens, 1, base_pos, window, bidirectional);
-    const float share = (float)s.tiles / kQ8CUs;
-    const float cost = 1.1f * (share > s.ct ? share : (float)s.ct) + 1.0f + 0.015f * s.wgs * D / 128;
-    return cost < whole ? s : PrefillSplit{};
+    return pf_split_choose(n_tokens, n_heads, n_kv_heads, base_pos, window, bidirectional, BM, BN, kQ8CUs, 1, whole,
+                           kQ8CUs, 0.015f * D / 128);
 }
 
 }  // namespace

@@ -14,6 +14,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 namespace gr {
 
 struct PrefillSplit {
@@ -87,36 +89,66 @@ inline void pf_split_carve(PrefillSplit& s, int n_kv, void* ws) {
 
 // The smallest piece of at least min_ct tiles whose workgroups all fit the
 // `slots` the GPU holds at once (0 splits if there is none worth having: pieces
-// as long as the blocks).
+// as long as the blocks).  Both counts only fall as pieces grow: the piece is found by
+// bisection, over block lengths computed once.
 inline PrefillSplit pf_split_plan(int n_tokens, int n_heads, int n_kv, int p0, int window, int bidirectional, int bm,
                                   int bn, int slots, int min_ct) {
     PrefillSplit s;
     const int kv_mul = n_heads / n_kv;
     s.bm = bm, s.bn = bn;
     s.n_qb = (int)(((int64_t)n_tokens * kv_mul + bm - 1) / bm);
-    auto tiles = [&](int qb) { return pf_split_tiles(qb, bm, bn, n_tokens, kv_mul, p0, window, bidirectional); };
+    if ((int64_t)s.n_qb * n_kv >= slots) return s;  // one piece a block fills the slots
+    std::vector<int> tiles(s.n_qb);
     int longest = 0;
     int64_t total = 0;
     for (int qb = 0; qb < s.n_qb; qb++) {
-        const int t = tiles(qb);
+        const int t = pf_split_tiles(qb, bm, bn, n_tokens, kv_mul, p0, window, bidirectional);
+        tiles[qb] = t;
         longest = t > longest ? t : longest;
         total += t;
     }
-    int ct = (int)((total * n_kv + slots - 1) / slots);
-    if (ct < min_ct) ct = min_ct;
-    for (; ct < longest; ct++) {
-        int64_t wgs = 0;
-        for (int qb = 0; qb < s.n_qb; qb++) wgs += (tiles(qb) + ct - 1) / ct;
-        const int n = (longest + ct - 1) / ct;
-        if (wgs * n_kv <= slots && (int64_t)s.n_qb * n_kv * n <= kPfSplitSlots * (int64_t)slots) {
-            s.ct = ct;
-            s.tiles = total * n_kv;
-            s.wgs = (int)(wgs * n_kv);
-            s.n_splits = n;
-            return s;
-        }
+    auto pieces = [&](int ct) {  // workgroups per KV head
+        int64_t n = 0;
+        for (int t : tiles) n += (t + ct - 1) / ct;
+        return n;
+    };
+    auto fits = [&](int ct) {
+        return pieces(ct) * n_kv <= slots &&
+               (int64_t)s.n_qb * n_kv * ((longest + ct - 1) / ct) <= kPfSplitSlots * (int64_t)slots;
+    };
+    int lo = (int)((total * n_kv + slots - 1) / slots), hi = longest;  // pieces of `longest` fit
+    if (lo < min_ct) lo = min_ct;
+    while (lo < hi) {
+        const int ct = lo + (hi - lo) / 2;
+        if (fits(ct)) hi = ct;
+        else lo = ct + 1;
     }
+    if (lo >= longest) return s;
+    s.ct = lo;
+    s.tiles = total * n_kv;
+    s.wgs = (int)(pieces(lo) * n_kv);
+    s.n_splits = (longest + lo - 1) / lo;
     return s;
+}
+
+// The plan if it is worth having against an unsplit launch that takes `whole` tiles of
+// time (its longest workgroup): at least one piece and its share of all tiles on `cus`
+// CUs, 1.1 for the uneven finish, a tile for the combine launch and per_wg per
+// workgroup for its partials.  Most launches that lose show it without a plan, by the keys
+// their rows see and a piece per block (a plan of 8192 tokens costs the host some us).
+inline PrefillSplit pf_split_choose(int n_tokens, int n_heads, int n_kv, int p0, int window, int bidirectional, int bm,
+                                    int bn, int slots, int min_ct, float whole, int cus, float per_wg) {
+    const int64_t n_qb = ((int64_t)n_tokens * (n_heads / n_kv) + bm - 1) / bm;
+    int64_t seen = 0;  // keys that the tokens see, causal (an image block's see more)
+    const int64_t n = n_tokens, in = window > 0 ? (window > p0 ? (window - p0 < n ? window - p0 : n) : 0) : n;
+    seen = in * p0 + in * (in + 1) / 2 + (n - in) * window;
+    const float least = 1.1f * ((float)(seen * n_heads) / ((float)bm * bn * cus)) + 1.0f + per_wg * (float)(n_qb * n_kv);
+    if (least * 0.999f >= whole) return {};
+    const PrefillSplit s = pf_split_plan(n_tokens, n_heads, n_kv, p0, window, bidirectional, bm, bn, slots, min_ct);
+    if (s.n_splits == 0) return s;
+    const float share = (float)s.tiles / cus;
+    const float cost = 1.1f * (share > s.ct ? share : (float)s.ct) + 1.0f + per_wg * s.wgs;
+    return cost < whole ? s : PrefillSplit{};
 }
 
 }  // namespace gr
