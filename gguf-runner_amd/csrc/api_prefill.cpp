@@ -97,13 +97,22 @@ size_t prefill_f16_copy_bytes(const gr_prefill_args* a) {
     return align_up((size_t)rows * a->n_kv_heads * a->head_dim * 2, 256);
 }
 
+PrefillSplit prefill_split(const gr_prefill_args* a) {
+    return prefill_split_plan(a->n_tokens, a->n_heads, a->n_kv_heads, a->head_dim, a->base_pos, a->window,
+                              a->bidirectional ? 1 : 0);
+}
+
 // [partials of a key-split launch][staging][K copy][V copy][flag, 256 B] for bf16,
-// [partials][staging] for f16.  The partials take the same room in every call, split
-// or not: a workspace sized for the longest chunk then also holds the shorter
-// chunks, which are the ones that split.
-size_t prefill_part_bytes(const gr_prefill_args* a) { return align_up(prefill_split_ws_bytes(a->head_dim), 256); }
-size_t prefill_ws_total(const gr_prefill_args* a) {
-    const size_t n = prefill_part_bytes(a) + prefill_stage_bytes(a);
+// [partials][staging] for f16.  In a caller's workspace the partials take the same room in
+// every call, split or not: one sized for the longest chunk then also holds the shorter
+// chunks, which are the ones that split.  The run state sizes each call (own_size): the
+// partials of its plan.
+size_t prefill_part_bytes(const gr_prefill_args* a, const PrefillSplit& split, bool own_size) {
+    return align_up(own_size ? pf_split_part_bytes(split, a->n_kv_heads, a->head_dim) : prefill_split_ws_bytes(a->head_dim),
+                    256);
+}
+size_t prefill_ws_total(const gr_prefill_args* a, bool own_size) {
+    const size_t n = prefill_part_bytes(a, own_size ? prefill_split(a) : PrefillSplit{}, own_size) + prefill_stage_bytes(a);
     if (a->dtype != GR_DTYPE_BF16) return n;
     return n + 2 * prefill_f16_copy_bytes(a) + 256;
 }
@@ -124,8 +133,9 @@ uint32_t next_f16_epoch() {
 
 // in_dtype: element type of a->q / a->k / a->v (the public entry point uses
 // a->dtype; the run-state path stages the reference's f32 rows directly).
-// feed: the run-state path's rows still on their way (null: all there).
-int prefill_enqueue_ex(const gr_prefill_args* a, int in_dtype, hipStream_t st, const PrepFeed* feed) {
+// feed: the run-state path's rows still on their way (null: all there).  own_size: the
+// workspace is prefill_ws_bytes(a, true) bytes.
+int prefill_enqueue_ex(const gr_prefill_args* a, int in_dtype, hipStream_t st, const PrepFeed* feed, bool own_size) {
     int rc = check_prefill(a);
     if (rc) return rc;
     if (a->n_tokens == 0) return GR_OK;
@@ -155,10 +165,9 @@ int prefill_enqueue_ex(const gr_prefill_args* a, int in_dtype, hipStream_t st, c
     pp.v = a->v;
     pp.q_row_stride = (int64_t)a->n_heads * a->head_dim;
     pp.kv_row_stride = (int64_t)a->n_kv_heads * a->head_dim;
-    PrefillSplit split = prefill_split_plan(a->n_tokens, a->n_heads, a->n_kv_heads, a->head_dim, a->base_pos, a->window,
-                                            a->bidirectional ? 1 : 0);
+    PrefillSplit split = prefill_split(a);
     pf_split_carve(split, a->n_kv_heads, a->workspace);
-    char* const stage = (char*)a->workspace + prefill_part_bytes(a);
+    char* const stage = (char*)a->workspace + prefill_part_bytes(a, split, own_size);
     // a split launch's workgroups each read their rows' Q: prepared once, by the prep pass
     const bool fused = split.n_splits == 0 && prefill_fused_q(a);
     const bool bf16 = a->dtype == GR_DTYPE_BF16;
@@ -256,9 +265,9 @@ int prefill_enqueue_ex(const gr_prefill_args* a, int in_dtype, hipStream_t st, c
     return GR_OK;
 }
 
-size_t prefill_ws_bytes(const gr_prefill_args* a) {
+size_t prefill_ws_bytes(const gr_prefill_args* a, bool own_size) {
     if (!a || a->n_tokens < 0 || a->n_heads <= 0 || a->head_dim <= 0) return 0;
-    return prefill_ws_total(a);
+    return prefill_ws_total(a, own_size);
 }
 
 int rope_freqs_host(float theta, int rope_dim, float* out) {
@@ -275,11 +284,11 @@ int rope_freqs_host(float theta, int rope_dim, float* out) {
 
 extern "C" {
 
-size_t gr_prefill_workspace_size(const gr_prefill_args* a) { return gr::prefill_ws_bytes(a); }
+size_t gr_prefill_workspace_size(const gr_prefill_args* a) { return gr::prefill_ws_bytes(a, false); }
 
 int gr_prefill_attention(const gr_prefill_args* a, void* stream) {
     gr::clear_error();
-    return gr::prefill_enqueue_ex(a, a ? a->dtype : 0, (hipStream_t)stream, nullptr);
+    return gr::prefill_enqueue_ex(a, a ? a->dtype : 0, (hipStream_t)stream, nullptr, false);
 }
 
 int gr_rope_freqs(float theta, int32_t rope_dim, float* freqs_out) {

@@ -347,8 +347,8 @@ int validate_config(const gr_attn_config* c) {
 
 }  // namespace
 
-int prefill_enqueue_ex(const gr_prefill_args* a, int in_dtype, hipStream_t st, const PrepFeed* feed);
-size_t prefill_ws_bytes(const gr_prefill_args* a);
+int prefill_enqueue_ex(const gr_prefill_args* a, int in_dtype, hipStream_t st, const PrepFeed* feed, bool own_size);
+size_t prefill_ws_bytes(const gr_prefill_args* a, bool own_size);
 int decode_enqueue_ex(const gr_decode_args* a, const int32_t* seq_slot, hipStream_t st);
 int deltanet_enqueue(const gr_deltanet_args* a, hipStream_t st);
 size_t deltanet_ws(const gr_deltanet_args* a);
@@ -857,6 +857,7 @@ static int prefill_rows(gr_run_state* s, int32_t seq, int32_t layer, int64_t bas
         a.window = (int32_t)w;
         a.rope_mode = s->cfg.rope_mode;
         a.rope_dim = s->rope_dim;
+        a.bidirectional = block ? 1 : 0;
         return a;
     };
     auto q8_split = [&](int n, int64_t pos0) {
@@ -872,7 +873,7 @@ static int prefill_rows(gr_run_state* s, int32_t seq, int32_t layer, int64_t bas
         const int r0 = cut[pc], n = cut[pc + 1] - r0;
         if (mfma) {
             const gr_prefill_args a = pf_args(n, base_pos + r0);
-            scratch = std::max(scratch, prefill_ws_bytes(&a) + 256);
+            scratch = std::max(scratch, prefill_ws_bytes(&a, true) + 256);
             continue;
         }
         pst[pc].assign(starts.begin() + r0, starts.begin() + r0 + n);
@@ -967,7 +968,7 @@ static int prefill_rows(gr_run_state* s, int32_t seq, int32_t layer, int64_t bas
         float* xi = xo + (size_t)r0 * s->q_dim;
         if (mfma) {
             gr_prefill_args a = pf_args(n, pos0);
-            const size_t ws = prefill_ws_bytes(&a);
+            const size_t ws = prefill_ws_bytes(&a, true);
             const bool swa = is_swa_layer(s, layer);
             a.rope_scale = swa ? s->cfg.rope_scale_local : s->cfg.rope_scale_global;
             a.rope_freqs = (s->cfg.is_gemma3 && swa) ? s->freqs_swa : s->freqs;
@@ -985,8 +986,7 @@ static int prefill_rows(gr_run_state* s, int32_t seq, int32_t layer, int64_t bas
             a.cache_row_stride = s->kv_dim;
             a.out = xi;
             a.workspace = cw.take<char>(ws);
-            a.bidirectional = block ? 1 : 0;
-            return prefill_enqueue_ex(&a, GR_DTYPE_F32, s->stream, fp);
+            return prefill_enqueue_ex(&a, GR_DTYPE_F32, s->stream, fp, true);
         }
         float* qp = cw.take<float>((size_t)n * s->q_dim);
         QkvPrepLaunch p = prep_for(s, layer, n, true, true);

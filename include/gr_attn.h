@@ -212,6 +212,13 @@ typedef struct gr_prefill_args {
     const float* v_bias;
 } gr_prefill_args;
 
+/* Bytes of a->workspace.  Every size holds the partial results of a launch that is cut
+ * along its keys (short chunks over long caches), whether or not this call is one: 36 MB at
+ * head_dim 64, 69 MB at 128, 68 MB at 256, and beyond them two bytes per element of q (bf16
+ * caches: and f16 copies of the cache rows that the chunk sees).  The calls of one stream
+ * can share a workspace of the largest of their sizes; an f16 one sized for the longest
+ * chunk serves the shorter ones too, wherever they start.  Sizes differ between versions
+ * of the library with the same GR_ATTN_ABI_VERSION: ask the one that runs. */
 size_t gr_prefill_workspace_size(const gr_prefill_args* a);
 int gr_prefill_attention(const gr_prefill_args* a, void* stream);
 

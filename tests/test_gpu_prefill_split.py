@@ -74,6 +74,23 @@ def test_split_prefill_gate_and_smaller_chunks_share_a_workspace(dev):
     assert torch.equal(out, outs[0])
 
 
+@pytest.mark.parametrize("kv_dtype", ["F16", "BF16"])
+def test_run_state_chunk_reserves_its_own_partials(dev, kv_dtype):
+    """A run state's short first chunk, which is not cut along its keys, takes device memory
+    for its rows (a few hundred KB), not for the partials that a cut one may have (69 MB at
+    head_dim 128).  Bound: 8 MB, the allocator's granularity and the mapped buffer's."""
+    from gguf_runner_amd import ffi, runtime as rt
+    p = rt.Config(n_layers=1, n_heads=32, n_kv_heads=8, head_dim=128, seq_len=64,
+                  kv_dtype=getattr(ffi, "DTYPE_" + kv_dtype), rope_mode=ffi.ROPE_NONE)
+    rows = [np.ones((16, w), np.float32) for w in (p.q_dim, p.kv_dim, p.kv_dim)]
+    rt.prefill_attention_chunk(p, rt.malloc_run_state(p), 0, 0, *rows)  # kernels loaded
+    s = rt.malloc_run_state(p)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    rt.prefill_attention_chunk(p, s, 0, 0, *rows)
+    assert free - torch.cuda.mem_get_info()[0] <= 8 << 20
+
+
 @pytest.mark.parametrize("block,h,g,d,m,hist,window,image", [
     (False, 32, 8, 128, 64, 900, None, False), (True, 16, 16, 128, 3, 1000, None, False),
     (False, 14, 2, 64, 50, 1100, 777, False), (True, 8, 4, 256, 40, 600, None, False),
