@@ -63,8 +63,7 @@ __global__ __launch_bounds__(kPrepThreads) void qkv_prep_kernel(const QkvPrepLau
     const int rows_per_token = p.n_heads + 2 * p.n_kv_heads;
     const int64_t pos = p.pos ? (int64_t)p.pos[i] : p.pos0 + i;
     const int half = p.rope_dim / 2;
-    const bool rope = p.rope_mode != GR_ROPE_NONE;
-    if (rope)
+    if (p.rope_mode != GR_ROPE_NONE)
         prep_rope_table(p, pos, wt * 64 + lane, WPT * 64, cs_t, sn_t,
                         p.rope_cs_out && tok_ok && blockIdx.y == 0 ? p.rope_cs_out + (size_t)i * half * 2 : nullptr);
     __syncthreads();
@@ -84,94 +83,9 @@ __global__ __launch_bounds__(kPrepThreads) void qkv_prep_kernel(const QkvPrepLau
         const int hrc = valid ? hr : rows_per_token - 1;
         const int kind = hrc < p.n_heads ? 0 : (hrc < p.n_heads + p.n_kv_heads ? 1 : 2);  // q, k, v
         const int head = kind == 0 ? hrc : (kind == 1 ? hrc - p.n_heads : hrc - p.n_heads - p.n_kv_heads);
-        const bool skip = !valid || (kind == 0 && p.q_out == nullptr);
-        float x[8];
-        // prep_row's body (qkv_row.hpp), in place: inlined from the function it takes 88
-        // registers instead of 77, five waves per SIMD instead of six, and the pass over
-        // 8192 tokens 28 us instead of 21 (32 / 8 heads, d128; 8 / 4 heads of d256 67 and 50)
-        const void* src = kind == 0 ? p.q : (kind == 1 ? p.k : p.v);
-        const int64_t rs = kind == 0 ? p.q_row_stride : p.kv_row_stride;
-        if (!skip) load8(src, (size_t)i * rs + (size_t)head * D + c8, p.in_dtype, x);
-        else
-#pragma unroll
-            for (int e = 0; e < 8; e++) x[e] = 0.0f;
-        // Qwen2 attention biases, before the norm (qkv_bias_and_norm, inference.rs:2545-2559)
-        const float* bias = kind == 0 ? p.q_bias : (kind == 1 ? p.k_bias : p.v_bias);
-        if (bias && !skip) {
-            float bv[8];
-            load8(bias, (size_t)head * D + c8, GR_DTYPE_F32, bv);
-#pragma unroll
-            for (int e = 0; e < 8; e++) x[e] += bv[e];
-        }
-        if (kind != 2) {
-            // QK RMSNorm: ss = sum(x^2)/d + eps; x = w * ((1/sqrt(ss)) * x).
-            const float* w = kind == 0 ? p.q_norm : p.k_norm;
-            float ss = fmaf(x[0], x[0], x[1] * x[1]);
-#pragma unroll
-            for (int e = 2; e < 8; e++) ss = fmaf(x[e], x[e], ss);
-            ss = wave_sum<LPR>(ss);  // lanes of other rows never mix: groups are LPR-aligned
-            if (w) {
-                const float inv = 1.0f / sqrtf(ss / (float)D + p.eps);
-                float wv[8];
-                load8(w, c8, GR_DTYPE_F32, wv);
-#pragma unroll
-                for (int e = 0; e < 8; e++) x[e] = wv[e] * (inv * x[e]);
-            }
-            if (rope) {
-                if (p.rope_mode == GR_ROPE_ADJACENT) {
-                    // pairs (2j, 2j+1) sit inside the lane's 8 elements
-#pragma unroll
-                    for (int e = 0; e < 8; e += 2) {
-                        const int fi = (c8 + e) >> 1;
-                        const float cs = cs_t[fi], sn = sn_t[fi];
-                        const float v0 = x[e], v1 = x[e + 1];
-                        x[e] = v0 * cs - v1 * sn;
-                        x[e + 1] = v0 * sn + v1 * cs;
-                    }
-                } else if (p.rope_dim == D) {
-                    // NeoX pairs (i, i + D/2) of a fully rotated row: the partner
-                    // elements of this lane's 8 are the 8 of lane ^ (LPR/2), in the
-                    // same row's lane group
-                    const bool first = c8 < half;
-                    const int f0 = first ? c8 : c8 - half;
-                    float csv[8], snv[8];
-                    *(float4*)csv = *(const float4*)(cs_t + f0);
-                    *(float4*)(csv + 4) = *(const float4*)(cs_t + f0 + 4);
-                    *(float4*)snv = *(const float4*)(sn_t + f0);
-                    *(float4*)(snv + 4) = *(const float4*)(sn_t + f0 + 4);
-#pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        const float other = __shfl_xor(x[e], LPR / 2, 64);
-                        // (v0, v1) -> (v0*c - v1*s, v0*s + v1*c)
-                        x[e] = first ? fmaf(-other, snv[e], x[e] * csv[e]) : fmaf(other, snv[e], x[e] * csv[e]);
-                    }
-                } else {
-                    // NeoX pairs (i, i + rope_dim/2) of a partial rotation live in
-                    // other lanes: stage the row
-#pragma unroll
-                    for (int e = 0; e < 8; e++) rb[c8 + e] = x[e];
-                    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        const int idx = c8 + e;
-                        if (idx >= p.rope_dim) continue;  // partial RoPE: tail untouched
-                        const bool first = idx < half;
-                        const int fi = first ? idx : idx - half;
-                        const float other = rb[first ? idx + half : idx - half];
-                        const float cs = cs_t[fi], sn = sn_t[fi];
-                        // (v0, v1) -> (v0*c - v1*s, v0*s + v1*c)
-                        x[e] = first ? x[e] * cs - other * sn : other * sn + x[e] * cs;
-                    }
-                    __builtin_amdgcn_wave_barrier();  // reads done before the next rows' stores
-                }
-            }
-            if (kind == 0 && p.gemma_q_scale) {
-                const float sc = 1.0f / sqrtf((float)D);
-#pragma unroll
-                for (int e = 0; e < 8; e++) x[e] *= sc;
-            }
-        }
-        if (skip) continue;
+        const PrepRow pr = prep_row<D>(p, i, kind, head, c8, cs_t, sn_t, rb);
+        const float (&x)[8] = pr.x;
+        if (!valid) continue;
         if (kind == 0) {
             const size_t ob = ((size_t)i * p.n_heads + head) * D + c8;
             float xs[8];

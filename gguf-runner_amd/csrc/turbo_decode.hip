@@ -361,12 +361,11 @@ __global__ __launch_bounds__(64) void turbo_token_kernel(const TurboToken f, con
     tq::wave_lds_sync();
     // every lane group of D / 8 lanes prepares the same row
     const int c8 = (lane % LPR) * 8;
-    float x8[8];
-    prep_row<D>(q, i, kind, head, false, c8, cs_t, sn_t, row_buf[lane / LPR], x8);
+    const PrepRow pr = prep_row<D>(q, i, kind, head, c8, cs_t, sn_t, row_buf[lane / LPR]);
     tq::wave_lds_sync();  // (a partial rotation's reads of row_buf precede the stores)
     if (lane < LPR) {
 #pragma unroll
-        for (int e = 0; e < 8; e++) row_buf[0][c8 + e] = kind == 0 ? x8[e] * q.q_out_scale : x8[e];
+        for (int e = 0; e < 8; e++) row_buf[0][c8 + e] = kind == 0 ? pr.x[e] * q.q_out_scale : pr.x[e];
     }
     tq::wave_lds_sync();
     float x[J];

@@ -416,7 +416,7 @@ def test_turbo_combine_many_partials(orc, dev, d):
 
 @pytest.mark.parametrize("d,n_heads,n_kv,rope,rope_dim,norm", [
     (128, 32, 8, "ROPE_NEOX", 0, True), (128, 40, 4, "ROPE_NEOX", 48, False),
-    (64, 32, 8, "ROPE_ADJACENT", 0, False), (64, 14, 2, "ROPE_NEOX", 0, True),
+    (128, 32, 8, "ROPE_ADJACENT", 0, True), (64, 32, 8, "ROPE_ADJACENT", 0, False), (64, 14, 2, "ROPE_NEOX", 0, True),
     (256, 16, 4, "ROPE_NEOX", 64, True), (256, 8, 4, "ROPE_NONE", 0, True)])
 def test_turbo_token_kernel_equals_passes(dev, d, n_heads, n_kv, rope, rope_dim, norm):
     """The same decode steps as one batch of more than 3072 head rows (preparation,
