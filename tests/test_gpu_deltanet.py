@@ -226,6 +226,58 @@ def test_deltanet_bf16_scan_product_rounding(dev):
     assert rel <= 2.0 ** -23, np.log2(rel)
 
 
+def _substitution(A):
+    """(I + A)^-1 of strictly lower f32 matrices [n][64][64] by forward substitution in f32, each
+    row's sum as chains of four terms summed in a tree."""
+    n = A.shape[0]
+    X = np.zeros_like(A)
+    for t in range(64):
+        p = (A[:, t, :, None] * X).reshape(n, 16, 4, 64).astype(np.float32)
+        c = ((p[:, :, 0] + p[:, :, 1]) + p[:, :, 2]) + p[:, :, 3]
+        while c.shape[1] > 1:
+            c = c[:, 0::2] + c[:, 1::2]
+        X[:, t] = -c[:, 0]
+        X[:, t, t] += np.float32(1)
+    return X
+
+
+@pytest.mark.parametrize("fmt", ["F32", "F16"])
+def test_deltanet_prep_inverse_is_as_close_as_substitution(orc, dev, fmt):
+    """T = (I + A)^-1 of the prep, read from the workspace's blocks, against 64 bits: at most 1.7
+    times as far off as f32 substitution with tree sums (1.45 times with the prep's sums
+    done on the CPU; 2.4 times with one chain over each block row's terms).  Keys whose
+    products are exact (first element 1, a few of +-1/8), no decay and betas of 8 bits make
+    A itself exact; T is then far from I."""
+    from gguf_runner_amd import ops
+    H, d, T = 8, 128, 512
+    rng = np.random.default_rng(21)
+    k = rng.integers(-1, 2, (T, H, d)) * (rng.random((T, H, d)) < 0.15) / 8.0
+    k[:, :, 0] = 1
+    beta = rng.integers(32, 224, (T, H)) / 256.0
+    dt = torch.float32 if fmt == "F32" else torch.float16
+    row = lambda x: torch.from_numpy(x).to(dev, dt)
+    call = ops.DeltaNetCall(row(np.zeros_like(k)), row(k), row(np.zeros_like(k)), torch.zeros((T, H), device=dev),
+                            torch.from_numpy(beta.astype(np.float32)).to(dev), torch.zeros((H, d, d), device=dev),
+                            torch.empty((T, H, d), device=dev), l2norm=False, algo=2)
+    call()
+    torch.cuda.synchronize()
+    first = -call.ws.data_ptr() % 256 + -(-32 * H // 256) * 256
+    blocks = call.ws.cpu().numpy()[first:first + T // 64 * H * 22528].view(np.float32).reshape(T // 64, H, 5632)
+    m, c = np.arange(16)[:, None], np.arange(16)[None]
+    at = (4 * m + ((c >> 2) ^ ((m >> 2) & 3))) * 4 + (c & 3)
+    got = np.zeros((T // 64, H, 64, 64), np.float32)
+    for r in range(4):
+        for q in range(r + 1):
+            got[:, :, 16 * r:16 * r + 16, 16 * q:16 * q + 16] = blocks[:, :, 256 * (r * (r + 1) // 2 + q) + at]
+    kk = k.reshape(T // 64, 64, H, d).transpose(0, 2, 1, 3)
+    A = np.tril(beta.reshape(T // 64, 64, H).transpose(0, 2, 1)[..., None] * (kk @ kk.transpose(0, 1, 3, 2)), -1)
+    assert np.array_equal(A, A.astype(np.float32))
+    want = np.linalg.inv(np.eye(64) + A)
+    off = lambda x: np.linalg.norm(x - want, axis=(2, 3)) / np.linalg.norm(want, axis=(2, 3))
+    sub = _substitution(A.reshape(-1, 64, 64).astype(np.float32)).reshape(want.shape)
+    assert off(got).mean() <= 1.7 * off(sub).mean(), (off(got).mean(), off(sub).mean())
+
+
 @pytest.mark.parametrize("d,algo,fmt_name", [(64, 1, "F32"), (64, 0, "BF16"), (256, 1, "F32"), (256, 2, "F16")])
 def test_deltanet_state_sizes_64_and_256(orc, dev, d, algo, fmt_name):
     """State sizes other than 128 (the reference takes any ssm_state_size, math.rs:566):
