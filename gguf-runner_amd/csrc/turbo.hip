@@ -18,6 +18,8 @@
 // reference for the same f32 row (no FMA contraction in this file).
 #pragma clang fp contract(off)
 
+#include <type_traits>
+
 #include "gr_common.hpp"
 #include "gr_internal.hpp"
 #include "stream_sched.hpp"
@@ -240,7 +242,7 @@ hipError_t launch_turbo_write(const TurboWriteLaunch& p, hipStream_t st) {
 template <int D, int WPH>
 __global__ __launch_bounds__(256) void turbo_combine_kernel(const DecodeLaunch p) {
     static_assert(WPH == 1 || WPH == 4, "a wave or the workgroup per head");
-    constexpr int J = D / 64, U = 8;
+    constexpr int J = D / 64;
     __shared__ float wsh_all[4][64];
     __shared__ float part[WPH > 1 ? 3 : 1][2 * J + 1][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -280,30 +282,33 @@ __global__ __launch_bounds__(256) void turbo_combine_kernel(const DecodeLaunch p
         wsh[lane] = w;
         tq::wave_lds_sync();  // the wave's weights visible to all its lanes
         const float* o = p.ws_o + (part0 + c0) * 2 * D;
-        int i = 0;
-        for (; i + U <= nc; i += U) {  // U partials' loads in flight together
+        // partials i .. i + U - 1, their loads in flight together; past the end the last one's
+        // again, not counted
+        auto take = [&](auto u_c, int i) {
+            constexpr int U = decltype(u_c)::value;
             float ob[U][J], orr[U][J];
 #pragma unroll
-            for (int u = 0; u < U; u++)
+            for (int u = 0; u < U; u++) {
+                const int at = min(i + u, nc - 1) * 2 * D + lane;
 #pragma unroll
                 for (int j = 0; j < J; j++) {
-                    ob[u][j] = o[(i + u) * 2 * D + lane + 64 * j];
-                    orr[u][j] = o[(i + u) * 2 * D + D + lane + 64 * j];
+                    ob[u][j] = o[at + 64 * j];
+                    orr[u][j] = o[at + D + 64 * j];
                 }
-#pragma unroll
-            for (int u = 0; u < U; u++)
-#pragma unroll
-                for (int j = 0; j < J; j++) {
-                    b[j] += ob[u][j] * wsh[i + u];
-                    r[j] += orr[u][j] * wsh[i + u];
-                }
-        }
-        for (; i < nc; i++)
-#pragma unroll
-            for (int j = 0; j < J; j++) {
-                b[j] += o[i * 2 * D + lane + 64 * j] * wsh[i];
-                r[j] += o[i * 2 * D + D + lane + 64 * j] * wsh[i];
             }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const bool in = i + u < nc;  // (a select: behind a branch the loads would follow each other)
+#pragma unroll
+                for (int j = 0; j < J; j++) {
+                    b[j] += (in ? ob[u][j] : 0.0f) * wsh[i + u];
+                    r[j] += (in ? orr[u][j] : 0.0f) * wsh[i + u];
+                }
+            }
+        };
+        int i = 0;
+        for (; nc - i > 4; i += 8) take(std::integral_constant<int, 8>{}, i);
+        if (i < nc) take(std::integral_constant<int, 4>{}, i);
         tq::wave_lds_sync();  // wsh reads done before the next chunk's stores
     }
     lt = wave_sum<64>(lt);
@@ -347,8 +352,9 @@ __global__ __launch_bounds__(256) void turbo_combine_kernel(const DecodeLaunch p
 }
 
 // More than kTurboCombineWide partials per head possible: a workgroup per head.
-// MI355X, us of this kernel: 2 x 32768 keys, 32 / 4 heads (about 32 partials) 7.8 -> 6.2;
-// a call of 1 x 8000 keys 20.8 -> 19.4 (32 / 4 heads), 20.3 -> 18.7 (32 / 8).
+// MI355X, us of a call, a wave -> a workgroup per head: 1 x 1100 keys (9 partials), 32 / 8
+// heads d128 16.7 -> 16.4, 14 / 2 heads d64 14.6 both; 1 x 3000 (24) 17.7 -> 16.7 and 15.2 -> 14.8;
+// 1 x 8000 (32) 19.7 -> 18.1 and 16.4 -> 15.8; 2 x 32768 keys, 32 / 4 heads 37.6 -> 35.2.
 constexpr int kTurboCombineWide = 8;
 
 template <int D>

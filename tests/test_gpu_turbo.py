@@ -414,6 +414,19 @@ def test_turbo_combine_many_partials(orc, dev, d):
         assert not got[2].any()
 
 
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_turbo_combine_takes_every_count_of_partials(orc, dev, d):
+    """Partials are taken in batches of eight and four, the last one partly past the end: every
+    count from 1 to 8 in one call (a wave per head), 1 to 16 and 17 to 32 in others (a
+    workgroup per head, a quarter of them to each wave)."""
+    for lo, hi in ((1, 8), (1, 16), (17, 32)):
+        n = hi - lo + 1
+        got, ref = _decode_case(orc, dev, n_heads=4, n_kv=2, d=d, starts=[0] * n,
+                                ends=[128 * c - 3 for c in range(lo, hi + 1)], seq_len=128 * hi, seed=d + hi)
+        err = np.abs(got - ref).reshape(n, -1).max(1)
+        assert (err <= TOL).all(), dict(enumerate(err, lo))
+
+
 @pytest.mark.parametrize("d,n_heads,n_kv,rope,rope_dim,norm", [
     (128, 32, 8, "ROPE_NEOX", 0, True), (128, 40, 4, "ROPE_NEOX", 48, False),
     (128, 32, 8, "ROPE_ADJACENT", 0, True), (64, 32, 8, "ROPE_ADJACENT", 0, False), (64, 14, 2, "ROPE_NEOX", 0, True),
