@@ -933,7 +933,7 @@ static int prefill_rows(gr_run_state* s, int32_t seq, int32_t layer, int64_t bas
         // heads: four pieces 2-5% slower, the launches cost what the overlap gives.)  Not
         // into memory of the buffer that no call has used yet: the host's first touch of its
         // pages bounds that copy, which two copy threads share and one thread feeding does
-        // not (first call of a state with a new buffer 1000 us, fed 1100).
+        // not (first call of a state with a new buffer 960 us, fed 1084).
         const size_t bytes = qb + 2 * kb;
         const int n_feed = bytes < (size_t(5) << 18) ? 1 : (int)std::min<size_t>({4, bytes / (size_t(3) << 17), (size_t)m});
         const bool fed = n_feed > 1 && s->mapped_used >= bytes;

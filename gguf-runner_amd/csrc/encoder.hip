@@ -309,10 +309,12 @@ __global__ __launch_bounds__(kEmThreads, (DP <= 128 ? 2 : 1)) void encoder_mfma_
 // row-major [key][dim]; the V^T operand comes from transposing reads
 // (ds_read_b64_tr_b16); Q is cut once per query row, P once per sub-tile.
 //
-// Bound by the matrix cores: 4096 tokens x 16 heads of 72 dims are 464 GFLOP of
-// piece products (515 with the padding), 394 us, 1307 TFLOP/s as issued, the rate a
-// large bf16 matrix product reaches on the same card (1304).  Before (four waves, one
-// chain of 30 dependent products per sub-tile, 96 padded dims in P V) 498 us.  What it
+// 4096 tokens x 16 heads of 72 dims are 464 GFLOP of piece products (515 with the
+// padding), 394 us, 1307 TFLOP/s as issued, the rate a large bf16 matrix product reaches
+// on the same card (1304), with the matrix cores busy in 0.62 of the cycles; the rest are
+// the softmax, the cutting into pieces and their waits, which two waves per SIMD hide
+// in part.  Before (four waves, one chain of 30 dependent products per sub-tile, 96
+// padded dims in P V) 498 us.  What it
 // came from: eight waves per tile 498 -> 438, the last 16 dims apart -> 430, both
 // sub-tiles' scores as two chains and the loads without branches -> 394 (alone on a
 // SIMD, 1000 tokens: 107 -> 82).  A wave priority around either product, or P V as
