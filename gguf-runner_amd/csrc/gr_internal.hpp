@@ -415,7 +415,7 @@ struct PrefillQ8Launch {
     PrefillSplit split;  // n_splits > 0: key-split launch and combine
 };
 
-// As prefill_split_plan; the partials take pf_split_part_bytes(plan, head_dim).
+// As prefill_split_plan; the partials take pf_split_part_bytes(plan, n_kv_heads, head_dim).
 PrefillSplit prefill_q8_split_plan(int n_tokens, int n_heads, int n_kv_heads, int head_dim, int base_pos, int window,
                                    int bidirectional);
 

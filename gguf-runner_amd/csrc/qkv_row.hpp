@@ -1,7 +1,6 @@
-// One head row of the per-token Q/K/V preparation for the Turbo cache's fused token
-// kernel (turbo_decode.hip): bias, QK RMSNorm, RoPE, Gemma q scale, the same f32 rows as
-// qkv_prep.hip, which has this body in place (there the function costs it a wave of
-// occupancy) and shares the loads and the RoPE table.
+// One head row of the per-token Q/K/V preparation: bias, QK RMSNorm, RoPE, Gemma q scale, in
+// f32.  The body of the preparation kernel (qkv_prep.hip) and of the Turbo cache's fused
+// token kernel (turbo_decode.hip), which must round a row alike.
 #pragma once
 
 #include "gr_common.hpp"
