@@ -907,7 +907,6 @@ static hipError_t launch_prefill_d(const PrefillLaunch& p, hipStream_t st) {
 // workgroups) 44.0 -> 36.4 us per call; at d128 (32 / 8 heads, S = 2048, 256
 // workgroups) the key halves were 1.5% slower than four waves.
 enum { kPfWaves8 = 8, kPfWaves4 = 4, kPfKeyHalves = 2 };
-constexpr int kPfCUs = 256;
 static int prefill_pick(const PrefillLaunch& p) {
     if (p.head_dim > 128) return kPfWaves4;
     const int n_qb8 = (p.n_tokens + 255) / 256, n_qb4 = (p.n_tokens + 127) / 128;
@@ -915,38 +914,13 @@ static int prefill_pick(const PrefillLaunch& p) {
     return p.head_dim == 64 && p.n_heads * ((n_qb4 + 1) / 2) <= kPfCUs ? kPfKeyHalves : kPfWaves4;
 }
 
-// Resident workgroups of the split kernels (two per CU at d <= 128, one at 256),
-// and the rows and keys of their tiles.
-struct PfSplitShape {
-    int slots, bm, bn;
-};
-static PfSplitShape pf_split_shape(int head_dim) {
-    if (head_dim == 64) return {2 * kPfCUs, 128, PfTile<64, 8, 2>::BN};
-    if (head_dim == 128) return {2 * kPfCUs, 128, PfTile<128, 4>::BN};
-    return {kPfCUs, 128, PfTile<256, 4>::BN};
-}
+static_assert(pf_split_shape(64).bn == PfTile<64, 8, 2>::BN && pf_split_shape(128).bn == PfTile<128, 4>::BN &&
+                  pf_split_shape(256).bn == PfTile<256, 4>::BN,
+              "the plan's tiles are the split kernels'");
 
-// Split or not: in tiles of 128 rows x BN keys, the unsplit launch takes its longest
-// pair of blocks (it has at most one workgroup per CU here); the split one as
-// pf_split_choose says, 0.03 (d128) per workgroup for its partials.  Fitted to 74
-// launches, 16 to 4096 tokens after 0 to 8000, five head shapes: the rule takes
-// the slower side by at most 4%.  MI355X, us per call (prep included), unsplit ->
-// split: 32 / 8 heads d128, 64 tokens after 4000 78.5 -> 29, 512 after 8000 302 -> 92,
-// 1500 after 8000 325 -> 267; 14 / 2 heads d64, 203 after 4000 83 -> 25, 1500 after
-// 8000 167 -> 80; 8 / 4 heads d256, 512 after 8000 543 -> 61.  Not split: 1500 tokens
-// from 0, d128 54 (63 split); 4096 from 0, d64 58 (73 split).
 PrefillSplit prefill_split_plan(int n_tokens, int n_heads, int n_kv_heads, int head_dim, int base_pos, int window,
                                 int bidirectional) {
-    const PfSplitShape sh = pf_split_shape(head_dim);
-    if (n_tokens <= 0) return {};
-    const int n_qb = (n_tokens - 1) / sh.bm + 1;
-    if ((int64_t)n_heads * ((n_qb + 1) / 2) > kPfCUs) return {};
-    auto block = [&](int qb) {
-        return pf_split_tiles(qb, sh.bm, sh.bn, n_tokens, 1, base_pos, window, bidirectional);
-    };
-    const float whole = (float)(block(n_qb - 1) + (n_qb > 1 ? block(0) : 0));
-    return pf_split_choose(n_tokens, n_heads, n_kv_heads, base_pos, window, bidirectional, sh.bm, sh.bn, sh.slots,
-                           128 / sh.bn, whole, kPfCUs, 0.03f * head_dim / 128);
+    return pf_split_16bit_plan(n_tokens, n_heads, n_kv_heads, head_dim, base_pos, window, bidirectional);
 }
 
 size_t prefill_split_ws_bytes(int head_dim) {

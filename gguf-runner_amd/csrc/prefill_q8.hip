@@ -576,7 +576,9 @@ constexpr int kQ8CUs = 256;  // resident workgroups: one per CU
 // gr_prefill_attention_chunk with its host rows, unsplit -> split: 32 / 8 heads
 // d128, 2 tokens after 4000 136 -> 42, 64 after 4000 285 -> 191, 512 after 4000 739 ->
 // 691; 14 / 2 heads d64, 64 after 4000 122 -> 59; 8 / 4 heads d256, 64 after 4000 297
-// -> 116.  Not split: chunks of 30 or fewer keys of history (equal within 3%).
+// -> 116.  At d64 one query block's launch must save two tiles for the combine launch (24
+// tokens after 300, 14 / 2 heads: 40.6, split 42.0).  Not split: chunks of 30 or fewer keys
+// of history (equal within 3%).
 template <int D>
 PrefillSplit q8_plan(int n_tokens, int n_heads, int n_kv_heads, int base_pos, int window, int bidirectional) {
     constexpr int BM = Q8Tile<D>::BM, BN = Q8Tile<D>::BN;
@@ -584,8 +586,14 @@ PrefillSplit q8_plan(int n_tokens, int n_heads, int n_kv_heads, int base_pos, in
     const int n_qb = (n_tokens - 1) / BM + 1;
     if ((int64_t)n_heads * n_qb > kQ8CUs) return {};
     const float whole = (float)pf_split_tiles(n_qb - 1, BM, BN, n_tokens, 1, base_pos, window, bidirectional);
+    PfSplitSaving saving;
+    if (D == 64 && n_qb == 1) {
+        saving.whole = (float)(pf_key_hi(base_pos, n_tokens - 1, n_tokens, bidirectional) -
+                               pf_key_lo(base_pos, 0, window, bidirectional)) / BN;
+        saving.launch = 2.0f;
+    }
     return pf_split_choose(n_tokens, n_heads, n_kv_heads, base_pos, window, bidirectional, BM, BN, kQ8CUs, 1, whole,
-                           kQ8CUs, 0.015f * D / 128);
+                           kQ8CUs, 0.015f * D / 128, saving);
 }
 
 }  // namespace

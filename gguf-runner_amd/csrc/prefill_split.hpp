@@ -131,13 +131,24 @@ inline PrefillSplit pf_split_plan(int n_tokens, int n_heads, int n_kv, int p0, i
     return s;
 }
 
+// What a cut must save in a launch's longest workgroup beyond the general cost below, in
+// tiles: the combine launch and its partials are a fixed cost that short caches do not earn.
+struct PfSplitSaving {
+    float whole = 1e30f;      // keys of the unsplit launch's longest workgroup, in tiles
+    float launch = 0.0f;      // the combine launch
+    float per_group = 0.0f;   // per 32 rows of partials
+    float partials = 0.0f;    // and at most for them
+};
+
 // The plan if it is worth having against an unsplit launch that takes `whole` tiles of
 // time (its longest workgroup): at least one piece and its share of all tiles on `cus`
 // CUs, 1.1 for the uneven finish, a tile for the combine launch and per_wg per
-// workgroup for its partials.  Most launches that lose show it without a plan, by the keys
-// their rows see and a piece per block (a plan of 8192 tokens costs the host some us).
+// workgroup for its partials; and `saving`.  Most launches that lose show it without a
+// plan, by the keys their rows see and a piece per block (a plan of 8192 tokens costs the
+// host some us).
 inline PrefillSplit pf_split_choose(int n_tokens, int n_heads, int n_kv, int p0, int window, int bidirectional, int bm,
-                                    int bn, int slots, int min_ct, float whole, int cus, float per_wg) {
+                                    int bn, int slots, int min_ct, float whole, int cus, float per_wg,
+                                    PfSplitSaving saving = {}) {
     const int64_t n_qb = ((int64_t)n_tokens * (n_heads / n_kv) + bm - 1) / bm;
     int64_t seen = 0;  // keys that the tokens see, causal (an image block's see more)
     const int64_t n = n_tokens, in = window > 0 ? (window > p0 ? (window - p0 < n ? window - p0 : n) : 0) : n;
@@ -148,7 +159,60 @@ inline PrefillSplit pf_split_choose(int n_tokens, int n_heads, int n_kv, int p0,
     if (s.n_splits == 0) return s;
     const float share = (float)s.tiles / cus;
     const float cost = 1.1f * (share > s.ct ? share : (float)s.ct) + 1.0f + per_wg * s.wgs;
-    return cost < whole ? s : PrefillSplit{};
+    const int64_t groups = ((int64_t)n_tokens * (n_heads / n_kv) + 31) / 32 * n_kv * s.n_splits;
+    const float written = saving.per_group * (float)groups;
+    const bool saves = saving.whole > (float)s.ct + saving.launch + (written < saving.partials ? written : saving.partials);
+    return cost < whole && saves ? s : PrefillSplit{};
+}
+
+// The 16-bit launches (prefill.hip).  Resident workgroups of the split kernels (two per CU
+// at d <= 128, one at 256), the rows and keys of their tiles, the cost per workgroup, and
+// what a cut of one query block's launch must save.
+constexpr int kPfCUs = 256;
+struct PfSplitShape {
+    int slots, bm, bn;
+    float per_wg, launch, per_group, partials;
+};
+constexpr PfSplitShape pf_split_shape(int head_dim) {
+    return head_dim == 64    ? PfSplitShape{2 * kPfCUs, 128, 128, 0.017f, 3.0f, 0.004f, 100.0f}
+           : head_dim == 128 ? PfSplitShape{2 * kPfCUs, 128, 64, 0.03f, 0.0f, 0.0125f, 5.0f}
+                             : PfSplitShape{kPfCUs, 128, 32, 0.06f, 3.0f, 0.0f, 0.0f};
+}
+
+// Split or not: in tiles of 128 rows x BN keys, the unsplit launch takes its longest
+// pair of blocks (it has at most one workgroup per CU here); the split one as
+// pf_split_choose says.  A launch of one query block is the shortest there is, and the
+// combine launch (3.7 us) and the partials must come out of its keys: PfSplitShape's
+// saving (the constants differ with the tile's time, and at d128 the unsplit kernel also
+// prepares Q); with two blocks or more, which the unsplit workgroups run in turn, 1.5
+// tiles.  Fitted to the launches that the general cost splits of 2241 (sixteen head
+// shapes, 2 to 2400 tokens after 0 to 5000, f16 and bf16): the side taken is slower than
+// the other by at most 7%, in 98 of 100 by less than 2%.  By the general cost alone 97 of
+// them were more than 2% slower split, up to 32%: 14 / 2 heads d64, 16 tokens after 250 11.3
+// us, split 14.9; 32 / 8 heads d128, 88 after 250 17.9, split 19.9.  (What it leaves whole
+// could still gain: 32 / 8 heads d128, 700 tokens after 130 42.6, split 34.2.)
+// MI355X, us per call (prep included), unsplit -> split: 32 / 8 heads d128, 64 tokens after
+// 4000 78.5 -> 29, 512 after 8000 302 -> 92, 1500 after 8000 325 -> 267; 14 / 2 heads d64,
+// 203 after 4000 83 -> 25, 1500 after 8000 167 -> 80; 8 / 4 heads d256, 512 after 8000 543
+// -> 61.  Not split: 1500 tokens from 0, d128 54 (63 split); 4096 from 0, d64 58 (73 split).
+inline PrefillSplit pf_split_16bit_plan(int n_tokens, int n_heads, int n_kv, int head_dim, int p0, int window,
+                                        int bidirectional) {
+    const PfSplitShape sh = pf_split_shape(head_dim);
+    if (n_tokens <= 0) return {};
+    const int n_qb = (n_tokens - 1) / sh.bm + 1;
+    if ((int64_t)n_heads * ((n_qb + 1) / 2) > kPfCUs) return {};
+    float whole = 0.0f, keys = 0.0f;
+    auto add = [&](int qb) {
+        const int last = (qb + 1) * sh.bm < n_tokens ? (qb + 1) * sh.bm - 1 : n_tokens - 1;
+        whole += (float)pf_split_tiles(qb, sh.bm, sh.bn, n_tokens, 1, p0, window, bidirectional);
+        keys += (float)(pf_key_hi(p0, last, n_tokens, bidirectional) - pf_key_lo(p0, qb * sh.bm, window, bidirectional));
+    };
+    add(n_qb - 1);
+    if (n_qb > 1) add(0);
+    const PfSplitSaving saving = n_qb > 1 ? PfSplitSaving{keys / sh.bn, 1.5f, 0.0f, 0.0f}
+                                          : PfSplitSaving{keys / sh.bn, sh.launch, sh.per_group, sh.partials};
+    return pf_split_choose(n_tokens, n_heads, n_kv, p0, window, bidirectional, sh.bm, sh.bn, sh.slots, 128 / sh.bn, whole,
+                           kPfCUs, sh.per_wg, saving);
 }
 
 }  // namespace gr

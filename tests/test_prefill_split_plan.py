@@ -164,3 +164,31 @@ def test_split_choice_is_the_first_fit_and_cheap(tmp_path):
                     str(src), "-o", str(exe)], check=True)
     out = subprocess.run([str(exe)], capture_output=True, text=True)
     assert out.returncode == 0, out.stdout
+
+
+# 16-bit launches timed both ways: (tokens, heads, KV heads, head_dim, tokens before, split).
+SHORT = [(16, 14, 2, 64, 250, 0), (40, 14, 2, 64, 400, 0), (88, 14, 2, 64, 504, 0), (40, 32, 8, 64, 250, 0),
+         (150, 14, 2, 64, 0, 0), (88, 32, 8, 128, 250, 0), (88, 32, 4, 128, 250, 0), (40, 8, 4, 256, 130, 0),
+         (88, 16, 2, 256, 130, 0), (256, 14, 2, 64, 0, 1), (150, 14, 2, 64, 130, 1), (40, 14, 2, 64, 1000, 1),
+         (203, 14, 2, 64, 3001, 1), (2, 32, 8, 128, 400, 1), (88, 32, 8, 128, 700, 1), (150, 32, 8, 128, 0, 1),
+         (64, 32, 8, 128, 4000, 1), (512, 8, 4, 256, 8000, 1), (40, 8, 4, 256, 400, 1), (4096, 14, 2, 64, 0, 0)]
+
+
+def test_split_of_16bit_launches_pays_for_its_combine(tmp_path):
+    """Short chunks over short caches, whose combine launch costs more than the cut saves (11.3
+    us whole, 14.9 cut: 16 tokens after 250, 14 / 2 heads of 64), stay whole; longer ones are cut."""
+    if not shutil.which("g++"):
+        pytest.skip("no host C++ compiler")
+    src = tmp_path / "short.cpp"
+    calls = "".join(f"    bad += check({m}, {h}, {g}, {d}, {p0}, {want});\n" for m, h, g, d, p0, want in SHORT)
+    src.write_text('#include "prefill_split.hpp"\n#include <cstdio>\n'
+                   "static int check(int m, int h, int g, int d, int p0, int want) {\n"
+                   "    const bool split = gr::pf_split_16bit_plan(m, h, g, d, p0, 0, 0).n_splits > 0;\n"
+                   "    if (split != (want != 0)) printf(\"%d tokens, %d / %d heads of %d after %d: split %d\\n\", m, h, g, d, p0, split);\n"
+                   "    return split != (want != 0);\n}\n"
+                   "int main() {\n    int bad = 0;\n" + calls + "    return bad;\n}\n")
+    exe = tmp_path / "short"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", f"-I{CSRC}",
+                    str(src), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout
