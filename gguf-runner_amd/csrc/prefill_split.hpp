@@ -185,11 +185,11 @@ constexpr PfSplitShape pf_split_shape(int head_dim) {
 // combine launch (3.7 us) and the partials must come out of its keys: PfSplitShape's
 // saving (the constants differ with the tile's time, and at d128 the unsplit kernel also
 // prepares Q); with two blocks or more, which the unsplit workgroups run in turn, 1.5
-// tiles.  Fitted to the launches that the general cost splits of 2241 (sixteen head
-// shapes, 2 to 2400 tokens after 0 to 5000, f16 and bf16): the side taken is slower than
-// the other by at most 7%, in 98 of 100 by less than 2%.  By the general cost alone 97 of
-// them were more than 2% slower split, up to 32%: 14 / 2 heads d64, 16 tokens after 250 11.3
-// us, split 14.9; 32 / 8 heads d128, 88 after 250 17.9, split 19.9.  (What it leaves whole
+// tiles.  Fitted to 2051 launches that the general cost splits (fifteen head shapes, 2 to
+// 2400 tokens after 0 to 5000, f16 and bf16): the side taken is slower than the other by
+// at most 7%, in 99 of 100 by less than 2%.  By the general cost alone 140 of them were more
+// than 2% slower split, up to 32%: 14 / 2 heads d64, 16 tokens after 250 11.3 us, split
+// 14.9; 32 / 8 heads d128, 88 after 250 17.9, split 19.9.  (What it leaves whole
 // could still gain: 32 / 8 heads d128, 700 tokens after 130 42.6, split 34.2.)
 // MI355X, us per call (prep included), unsplit -> split: 32 / 8 heads d128, 64 tokens after
 // 4000 78.5 -> 29, 512 after 8000 302 -> 92, 1500 after 8000 325 -> 267; 14 / 2 heads d64,
